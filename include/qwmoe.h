@@ -303,11 +303,22 @@ int qw_pack_bf16_tiles(const void* w, int64_t experts, int64_t out_features, int
  * QuantizedLinear.forward, src/quantization.py:71-72); x and out have
  * act_dtype (QW_F32, QW_BF16 or QW_F16); fp32 accumulation, quantised weights rounded
  * to act_dtype before the multiply.  max_rows_per_expert bounds every
- * expert's row count (0: rows); bf16 (fp16) with plain bf16 (fp16) weights and
- * in_features % 64 == 0 runs on the matrix cores. */
+ * expert's row count (0: rows); bf16 (fp16) with plain bf16 (fp16) or
+ * quantised weights and in_features % 64 == 0 runs on the matrix cores. */
 int qw_grouped_matmul(const void* x, int act_dtype, const void* w, int w_format, const float* scales, int64_t group,
                       int64_t experts, int64_t out_features, int64_t in_features, const int32_t* offsets,
                       int64_t rows, int64_t max_rows_per_expert, void* out, void* stream);
+
+/* One quantised matrix applied to every row, QuantizedLinear.forward
+ * (src/quantization.py:71-72): out[r] = x[r] @ w^T, w [out_features,
+ * in_features] as QW_I8 or QW_U4 with fp32 scales and group size `group`.  A
+ * few 16-bit rows stream the weights (exact codes times the fp32 scales);
+ * more run on the matrix cores with the weights rounded to act_dtype before
+ * the multiply.  Unlike qw_grouped_matmul it takes no row offsets, so a caller
+ * has nothing to copy to the device first. */
+int qw_quantized_matmul(const void* x, int act_dtype, const void* qweight, int w_format, const float* scales,
+                        int64_t group, int64_t out_features, int64_t in_features, int64_t rows, void* out,
+                        void* stream);
 
 /* The accumulation of the capacity-free static dispatch, replacing the loop
  * of TopKMoE._static_output (src/quantweave_moe_model.py:235-245):

@@ -38,8 +38,8 @@ __global__ __launch_bounds__(256) void ffn_generic_kernel(const void* __restrict
   __shared__ float xs[GB_M][GB_K + 1];
   __shared__ float os[GB_M][GB_N + 1];
   const int e = blockIdx.y;
-  // rows of expert e, clamped to the caller's buffers
-  const int r0 = max(offsets[e], 0), r1 = min(offsets[e + 1], max_rows);
+  // rows of expert e, clamped to the caller's buffers (no offsets: one expert, every row)
+  const int r0 = offsets ? max(offsets[e], 0) : 0, r1 = offsets ? min(offsets[e + 1], max_rows) : max_rows;
   if (r1 <= r0) return;
   const int tid = threadIdx.x;
   // GATEUP: tile covers 32 output columns: weight rows 0..31 gate, 32..63 up.

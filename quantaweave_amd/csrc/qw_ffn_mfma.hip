@@ -57,18 +57,15 @@
 // over the 8 XCDs, so block b runs on XCD b%8; all tiles of one expert are
 // given to one XCD and enumerated column-fastest, which keeps the expert's
 // activation rows (and a second row chunk's weights) in that XCD's L2.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
-#include "qw_ffn.h"
+#include "qw_mfma.h"
 
 namespace qw {
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));  // 16-bit operands (bf16 or fp16 bits)
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int MF_BK = 64;       // K slice: two MFMA K steps
 constexpr int MF_ROWB = 128;    // bytes per LDS row (64 bf16, no padding: swizzled)
@@ -110,92 +107,22 @@ constexpr int mf_stages(int subt) {
   return MF_LDS / stage >= 3 ? 3 : 2;
 }
 
-// s_waitcnt immediate waiting for vmcnt <= n only (expcnt, lgkmcnt left at max).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | (((N >> 4) & 3) << 14));
-}
-
 // 16-byte piece `piece` (0..7) of LDS row `row` is stored at physical piece
 // piece ^ ((row >> 1) & 7): the 16-row fragment reads of an MFMA (one logical
 // piece, rows 0..15) then touch 16 distinct bank groups.
 __device__ __forceinline__ int swz(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-// Barrier for the LDS ring: the slice's loads were already waited for with an
-// explicit vmcnt, so no fence is needed (a workgroup fence would wait for every
-// load still in flight, including the slices requested ahead).  The empty asm
-// statements keep the compiler from moving LDS accesses across the barrier.
-__device__ __forceinline__ void ring_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Weights of one projection for the kernel: bytes per expert and per stored
-// row; scales (quantised formats) per expert, per row, and the group size.
-struct MfW {
-  const char* w;
-  const float* scales;
-  int64_t expert_bytes, row_bytes, expert_scales;
-  int groups, group;
-};
-
-// One 16x16x32 MFMA step in the activation type: bf16, or fp16 bits carried
-// in the same 16-byte operand registers.
-template <int ACT>
-__device__ __forceinline__ f32x4 mfma_step(bf16x8 a, bf16x8 b, f32x4 c) {
-  if constexpr (ACT == QW_F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                                   0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Eight fp32 values rounded to the activation type, as 16-bit operand bits.
-template <int ACT>
-__device__ __forceinline__ bf16x8 pack_act8(const float (&f)[8]) {
-  if constexpr (ACT == QW_F16) {
-    f16x8 r;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = static_cast<_Float16>(pin_f32(f[i]));  // fp32 first, then RNE to fp16
-    return __builtin_bit_cast(bf16x8, r);
-  } else {
-    bf16x8 r;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = static_cast<__bf16>(f[i]);
-    return r;
-  }
-}
-
-// Eight int8 weights (bytes 0..7 = columns c..c+7) -> act(q * s).  The sign
-// bit flip stores u = q + 128; fma(u, s, -128 s) = q s rounded once.
+// Eight int8 weights (bytes 0..7 = columns c..c+7) -> act(q * s).
 template <int ACT>
 __device__ __forceinline__ bf16x8 dequant_i8(uint2 raw, float s) {
-  const uint32_t u0 = raw.x ^ 0x80808080u, u1 = raw.y ^ 0x80808080u;
-  const float c = -128.0f * s;
-  float f[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    f[i] = __builtin_fmaf(static_cast<float>((u0 >> (8 * i)) & 0xffu), s, c);
-    f[4 + i] = __builtin_fmaf(static_cast<float>((u1 >> (8 * i)) & 0xffu), s, c);
-  }
-  return pack_act8<ACT>(f);
+  return scale_bytes_seq<ACT>(raw.x ^ 0x80808080u, raw.y ^ 0x80808080u, s, -128.0f * s);
 }
 
 // Eight int4 weights (byte b: column c+2b in the low nibble, c+2b+1 in the
 // high one, each stored as q + 8) -> act(q * s).
 template <int ACT>
 __device__ __forceinline__ bf16x8 dequant_u4(uint32_t raw, float s) {
-  const uint32_t lo = raw & 0x0f0f0f0fu, hi = (raw >> 4) & 0x0f0f0f0fu;
-  const float c = -8.0f * s;
-  float f[8];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    f[2 * b] = __builtin_fmaf(static_cast<float>((lo >> (8 * b)) & 0xffu), s, c);
-    f[2 * b + 1] = __builtin_fmaf(static_cast<float>((hi >> (8 * b)) & 0xffu), s, c);
-  }
-  return pack_act8<ACT>(f);
+  return scale_bytes<ACT>(raw & 0x0f0f0f0fu, (raw >> 4) & 0x0f0f0f0fu, s, -8.0f * s);
 }
 
 template <int ACT, bool GATEUP, int SUBT, int WF>
@@ -586,20 +513,6 @@ __global__ __launch_bounds__(MF_THREADS) void ffn_mfma_kernel(
   }
 }
 
-// Kernel view of one stacked projection.
-MfW mf_view(int wf, const WView& v) {
-  const int64_t esize = wf == QW_I8 || wf == QW_U4 ? 1 : 2;  // QW_U4 strides are in bytes already
-  MfW m;
-  m.w = static_cast<const char*>(v.w);
-  m.scales = v.scales;
-  m.expert_bytes = v.expert_elems * esize;
-  m.row_bytes = v.row_stride * esize;
-  m.expert_scales = v.expert_scales;
-  m.groups = static_cast<int>(v.groups);
-  m.group = static_cast<int>(v.group > 0 ? v.group : 1);
-  return m;
-}
-
 template <int ACT, bool GATEUP, int SUBT, int WF>
 int launch_t(const void* x, const int32_t* row_index, const int32_t* offsets, int max_rows, const MfW& wa,
              const MfW& wb, int n_w, int K, const float* row_weight, void* out, int n_out, int experts,
@@ -651,15 +564,6 @@ int pick_subt(int64_t rows_cap) {
   return 10;
 }
 
-// The quantised projection suits the LDS stage: groups of whole MFMA K steps,
-// 16-byte aligned rows and base.
-bool quant_fits(const WView& v, int wf) {
-  const int64_t row_bytes = v.row_stride;  // int8: one byte per element; int4: bytes
-  return v.group > 0 && v.group % 32 == 0 && row_bytes % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(v.w) % 16 == 0 && reinterpret_cast<uintptr_t>(v.scales) % 4 == 0 &&
-         (wf == QW_I8 || wf == QW_U4);
-}
-
 }  // namespace
 
 int launch_ffn_mfma(const FfnArgs& a, hipStream_t stream, bool* handled) {
@@ -671,9 +575,14 @@ int launch_ffn_mfma(const FfnArgs& a, hipStream_t stream, bool* handled) {
     return QW_OK;
   if (a.d_model % 64 || a.d_ff % 64) return QW_OK;
   if (quant && !(quant_fits(a.gate, a.wfmt) && quant_fits(a.up, a.wfmt) && quant_fits(a.down, a.wfmt))) return QW_OK;
-  if (a.avg_rows < 16) return QW_OK;  // decode-sized: weight streaming kernels
   const int64_t rows_cap = a.row_cap > 0 ? a.row_cap : a.max_rows;
-  const int subt = pick_subt(rows_cap);
+  if (quant && likely_rows(a, 2.0) <= kQuantRows) return QW_OK;  // dequantised once per weight instead of twice
+  // An expert's second chunk reads all its weights again and, started last,
+  // costs a whole workgroup's time (T = 7000, capacity 274: 292 us in chunks
+  // of 256 rows against 248 us in chunks of 320): the bound where one chunk
+  // holds it, else room for 3.5 standard deviations (T = 512 without capacity:
+  // 163 us in chunks of 64 rows against 181 us in chunks of 320).
+  const int subt = pick_subt(rows_cap <= 320 ? rows_cap : likely_rows(a, 3.5));
   const int D = static_cast<int>(a.d_model), F = static_cast<int>(a.d_ff), E = static_cast<int>(a.experts);
   const int mr = static_cast<int>(a.max_rows);
   const MfW g = mf_view(a.wfmt, a.gate), u = mf_view(a.wfmt, a.up), dn = mf_view(a.wfmt, a.down);

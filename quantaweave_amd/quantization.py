@@ -89,11 +89,10 @@ class QuantizedLinear(nn.Module):
         rows = flat.size(0)
         out = torch.empty(rows, self.out_features, dtype=x.dtype, device=x.device)
         if rows:
-            offsets = torch.tensor([0, rows], dtype=torch.int32, device=x.device)
             scales = self.scales if self.scales.dtype == torch.float32 else self.scales.float()
-            _lib.call("qw_grouped_matmul", _hip.ptr(flat), act, _hip.ptr(self.qweight), self.w_format,
-                      _hip.ptr(scales.contiguous()), self.group_size, 1, self.out_features, self.in_features,
-                      _hip.ptr(offsets), rows, 0, _hip.ptr(out), _hip.stream(x.device))
+            qweight, scales = self.qweight.contiguous(), scales.contiguous()
+            _lib.call("qw_quantized_matmul", _hip.ptr(flat), act, _hip.ptr(qweight), self.w_format, _hip.ptr(scales),
+                      self.group_size, self.out_features, self.in_features, rows, _hip.ptr(out), _hip.stream(x.device))
         return out.reshape(*lead, self.out_features)
 
     def stored_bytes(self) -> int:
