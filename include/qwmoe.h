@@ -311,10 +311,9 @@ int qw_grouped_matmul(const void* x, int act_dtype, const void* w, int w_format,
 
 /* One quantised matrix applied to every row, QuantizedLinear.forward
  * (src/quantization.py:71-72): out[r] = x[r] @ w^T, w [out_features,
- * in_features] as QW_I8 or QW_U4 with fp32 scales and group size `group`.  A
- * few 16-bit rows stream the weights (exact codes times the fp32 scales);
- * more run on the matrix cores with the weights rounded to act_dtype before
- * the multiply.  Unlike qw_grouped_matmul it takes no row offsets, so a caller
+ * in_features] as QW_I8 or QW_U4 with fp32 scales and group size `group`;
+ * fp32 accumulation, the weights rounded to act_dtype before the multiply, on
+ * the matrix cores for 16-bit rows with in_features % 64 == 0.  Unlike qw_grouped_matmul it takes no row offsets, so a caller
  * has nothing to copy to the device first. */
 int qw_quantized_matmul(const void* x, int act_dtype, const void* qweight, int w_format, const float* scales,
                         int64_t group, int64_t out_features, int64_t in_features, int64_t rows, void* out,

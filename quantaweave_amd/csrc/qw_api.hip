@@ -652,16 +652,7 @@ int qw_quantized_matmul(const void* x, int act_dtype, const void* qweight, int w
   QW_REQUIRE(x && qweight && scales && out, "quantized_matmul pointers are required");
   const WView v = make_wview(w_format, qweight, scales, out_features, in_features, group);
   bool handled = false;
-  int st = QW_OK;
-  // A pass of the streaming kernels takes 4 rows and the whole matrix; the
-  // matrix-core kernel's time hardly depends on the rows until its grid fills
-  // the chip.  2048 x 7168, bf16 rows: int8 26 us streamed against 32 us at 16
-  // rows, 36 against 32 at 24; int4 29 against 34 us at 48, 36 against 34 at 64.
-  if (rows <= (w_format == QW_I8 ? 20 : 48)) {
-    st = stream_matmul(x, act_dtype, v, w_format, rows, out, as_stream(stream), &handled);
-    if (st || handled) return st;
-  }
-  st = quant_matmul(x, act_dtype, v, w_format, 1, nullptr, rows, rows, out, as_stream(stream), &handled);
+  const int st = quant_matmul(x, act_dtype, v, w_format, 1, nullptr, rows, rows, out, as_stream(stream), &handled);
   if (st || handled) return st;
   return grouped_matmul_generic(x, act_dtype, v, w_format, 1, nullptr, rows, out, as_stream(stream));
 }

@@ -8,7 +8,7 @@ namespace qw {
 struct FfnArgs {
   const void* x;             // activations [*, d_model] (act dtype)
   const int32_t* row_index;  // row s reads x[row_index[s]]; NULL: x[s]
-  const int32_t* offsets;    // [experts+1] row blocks per expert (device); NULL: one expert, every row
+  const int32_t* offsets;    // [experts+1] row blocks per expert (device)
   int64_t experts, d_model, d_ff, max_rows;
   int act, wfmt;
   WView gate, up, down;
@@ -77,8 +77,6 @@ int launch_ffn_quant(const FfnArgs& a, hipStream_t stream, bool* handled);
 // One quantised projection applied to grouped rows (offsets NULL: one matrix, every row).
 int quant_matmul(const void* x, int act, const WView& w, int wfmt, int64_t E, const int32_t* offsets, int64_t rows,
                  int64_t row_cap, void* out, hipStream_t stream, bool* handled);
-int stream_matmul(const void* x, int act, const WView& w, int wfmt, int64_t rows, void* out, hipStream_t stream,
-                  bool* handled);
 int launch_ffn_f32(const FfnArgs& a, hipStream_t stream, bool* handled);
 int grouped_matmul_f32(const float* x, const float* w, int64_t E, int64_t N, int64_t K, const int32_t* offsets,
                        int64_t rows, float* out, hipStream_t stream, bool* handled);

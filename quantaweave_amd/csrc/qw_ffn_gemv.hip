@@ -388,11 +388,6 @@ __device__ __forceinline__ uint32_t lds_addr(const char* p) {
 // per row), not all of them.  Wave-uniform result.
 __device__ __forceinline__ int nth_active_expert(const int32_t* __restrict__ offsets, int E, int max_rows, int j,
                                                  int* lo, int* hi) {
-  if (offsets == nullptr) {  // one expert holds every row
-    *lo = 0;
-    *hi = max_rows;
-    return j == 0 ? 0 : -1;
-  }
   const int lane = threadIdx.x % kWave;
   for (int c = 0; c < E; c += kWave) {
     const int e = c + lane;
@@ -735,11 +730,6 @@ struct QmfLds {
 // it has passes.  Wave-uniform result.
 __device__ __forceinline__ int nth_active_pass(const int32_t* __restrict__ offsets, int E, int max_rows, int j,
                                                int* lo, int* hi) {
-  if (offsets == nullptr) {  // one expert holds every row
-    *lo = 4 * j;
-    *hi = min(4 * j + 4, max_rows);
-    return 4 * j < max_rows ? 0 : -1;
-  }
   const int lane = threadIdx.x % kWave;
   for (int c = 0; c < E; c += kWave) {
     const int e = c + lane;
@@ -1395,41 +1385,6 @@ int launch_ffn_gemv(const FfnArgs& a, hipStream_t stream, bool* handled) {
     else if (a.wfmt == QW_BF16T) st = launch_fmt<QW_BF16, QW_BF16T>(a, stream);
     else st = launch_fmt<QW_BF16, QW_BF16>(a, stream);
   }
-  if (st) return st;
-  *handled = true;
-  return QW_OK;
-}
-
-// out = x . w^T of one quantised matrix on the weight-streaming kernels (every
-// pass of up to 4 rows, 2 for rows too long for the matrix-core kernel, streams
-// the whole matrix).
-int stream_matmul(const void* x, int act, const WView& w, int wfmt, int64_t rows, void* out, hipStream_t stream,
-                  bool* handled) {
-  *handled = false;
-  const int cw = wfmt == QW_U4 ? 32 : 16;
-  const int64_t K = w.cols;
-  if (!is_half(act) || !quantized(wfmt) || w.group % cw || K % cw || ceil_div(K / cw, 64) > 4) return QW_OK;
-  if (w.row_stride * (wfmt == QW_U4 ? 2 : 1) != K || rows > 4 * 65535) return QW_OK;
-  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w.w) | reinterpret_cast<uintptr_t>(w.scales)) & 15)
-    return QW_OK;
-  FfnArgs a{};
-  a.experts = 1;
-  a.max_rows = rows;
-  a.act = act;
-  a.wfmt = wfmt;
-  const int k = static_cast<int>(K), n = static_cast<int>(w.rows);
-  auto go = [&](auto act_c, auto wf_c) -> int {
-    constexpr int ACT = decltype(act_c)::value, WF = decltype(wf_c)::value;
-    if (K <= (WF == QW_I8 ? 2048 : 4096))
-      return launch_qmf<ACT, WF, false>(a, w, w, x, nullptr, k, n, nullptr, out, stream);
-    return launch_cpl<ACT, WF, false>(a, w, w, x, nullptr, k, n, nullptr, out, nullptr, nullptr, stream);
-  };
-  using I8 = std::integral_constant<int, QW_I8>;
-  using U4 = std::integral_constant<int, QW_U4>;
-  using BF = std::integral_constant<int, QW_BF16>;
-  using HF = std::integral_constant<int, QW_F16>;
-  const int st = act == QW_F16 ? (wfmt == QW_I8 ? go(HF{}, I8{}) : go(HF{}, U4{}))
-                               : (wfmt == QW_I8 ? go(BF{}, I8{}) : go(BF{}, U4{}));
   if (st) return st;
   *handled = true;
   return QW_OK;

@@ -61,6 +61,74 @@ __device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
   b = r[1];
 }
 
+// Exchange between the quarters of a wave: a slice's codes as loaded become
+// cw[t][s] (int4) or cw[t][2 s], [2 s + 1] (int8), the operand codes of step s;
+// its scales (one per lane, tile and slice; one per row: RS) become s4[t][s].
+template <int WF, int KS, bool RS, int DW, int STEPS>
+__device__ __forceinline__ void exchange(uint32_t (&cw)[QP_NT][DW], const float (&cs)[QP_NT],
+                                         float (&s4)[QP_NT][STEPS]) {
+  static_assert(STEPS == KS / 32, "MFMA steps of a slice");
+#pragma unroll
+  for (int t = 0; t < QP_NT; ++t) {
+    if constexpr (WF == QW_U4 && KS == 128) {
+      swap32(cw[t][0], cw[t][2]);
+      swap32(cw[t][1], cw[t][3]);
+      swap16(cw[t][0], cw[t][1]);
+      swap16(cw[t][2], cw[t][3]);
+    } else if constexpr (WF == QW_U4) {
+      swap16(cw[t][0], cw[t][1]);
+    } else {  // dwords (0, 1) and (2, 3) are the halves of the lane's 16 codes
+      swap16(cw[t][0], cw[t][2]);
+      swap16(cw[t][1], cw[t][3]);
+    }
+    if constexpr (RS) {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) s4[t][s] = cs[t];
+    } else {
+      uint32_t a = __float_as_uint(cs[t]), c = a;
+      if constexpr (KS == 128) {
+        swap32(a, c);
+        uint32_t a2 = a, c2 = c;
+        swap16(a, a2);
+        swap16(c, c2);
+        s4[t][0] = __uint_as_float(a);
+        s4[t][1] = __uint_as_float(a2);
+        s4[t][2] = __uint_as_float(c);
+        s4[t][3] = __uint_as_float(c2);
+      } else {
+        swap16(a, c);
+        s4[t][0] = __uint_as_float(a);
+        s4[t][1] = __uint_as_float(c);
+      }
+    }
+  }
+}
+
+// Tile t's weight operand of step s: act(q * scale) of 8 columns.
+template <int ACT, int WF, int DW>
+__device__ __forceinline__ bf16x8 weight_operand(const uint32_t (&c)[DW], int s, float scale) {
+  if constexpr (WF == QW_I8) {
+    return scale_bytes_seq<ACT>(c[2 * s] ^ 0x80808080u, c[2 * s + 1] ^ 0x80808080u, scale, -128.0f * scale);
+  } else {
+    const uint32_t r = c[s];
+    return scale_bytes<ACT>(r & 0x0f0f0f0fu, (r >> 4) & 0x0f0f0f0fu, scale, -8.0f * scale);
+  }
+}
+
+// Loads one tile's codes of a slice from p.
+template <int DW>
+__device__ __forceinline__ void load_codes(const char* p, uint32_t (&r)[DW]) {
+  if constexpr (DW == 4) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = v[i];
+  } else {
+    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+    r[0] = v[0];
+    r[1] = v[1];
+  }
+}
+
 // KS: K columns per slice (128 for int4 rows of whole 128-code pieces, else
 // 64).  SUB: 16-row sub-tiles of activations per workgroup.
 // RS: one scale per row.
@@ -151,18 +219,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
   constexpr int BL = QP_NT * (RS ? 1 : 2);  // loads per slice
   auto load_b = [&](int kt, uint32_t (&r)[QP_NT][DW], float (&f)[QP_NT]) {
 #pragma unroll
-    for (int t = 0; t < QP_NT; ++t) {
-      const char* p = b_src[t] + kt * (16 * DW);
-      if constexpr (DW == 4) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[t][i] = v[i];
-      } else {
-        const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-        r[t][0] = v[0];
-        r[t][1] = v[1];
-      }
-    }
+    for (int t = 0; t < QP_NT; ++t) load_codes<DW>(b_src[t] + kt * (16 * DW), r[t]);
     if constexpr (!RS) {
       const int step = kt * STEPS + step32;
       const int idx = group32 == 1 ? step : step / group32;
@@ -218,42 +275,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
       const int nstage = stage == 0 ? 2 : stage - 1;
       issue_a(next, nstage);
       load_b(next, raw[BUF], sc[BUF]);
-      // exchange between the quarters: cw[t][s] (int4) or cw[t][2s], [2s+1]
-      // (int8) become step s's operand codes; s4[t][s] its scales
-#pragma unroll
-      for (int t = 0; t < QP_NT; ++t) {
-        if constexpr (WF == QW_U4 && KS == 128) {
-          swap32(cw[t][0], cw[t][2]);
-          swap32(cw[t][1], cw[t][3]);
-          swap16(cw[t][0], cw[t][1]);
-          swap16(cw[t][2], cw[t][3]);
-        } else if constexpr (WF == QW_U4) {
-          swap16(cw[t][0], cw[t][1]);
-        } else {  // dwords (0, 1) and (2, 3) are the halves of the lane's 16 codes
-          swap16(cw[t][0], cw[t][2]);
-          swap16(cw[t][1], cw[t][3]);
-        }
-        if constexpr (RS) {
-#pragma unroll
-          for (int s = 0; s < STEPS; ++s) s4[t][s] = cs[t];
-        } else {
-          uint32_t a = __float_as_uint(cs[t]), c = a;
-          if constexpr (KS == 128) {
-            swap32(a, c);
-            uint32_t a2 = a, c2 = c;
-            swap16(a, a2);
-            swap16(c, c2);
-            s4[t][0] = __uint_as_float(a);
-            s4[t][1] = __uint_as_float(a2);
-            s4[t][2] = __uint_as_float(c);
-            s4[t][3] = __uint_as_float(c2);
-          } else {
-            swap16(a, c);
-            s4[t][0] = __uint_as_float(a);
-            s4[t][1] = __uint_as_float(c);
-          }
-        }
-      }
+      exchange<WF, KS, RS>(cw, cs, s4);
       const char* st = smem + stage * A_STAGE;
       stage = stage == 2 ? 0 : stage + 1;
       auto read_a = [&](int i, int s) {
@@ -264,15 +286,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
       for (int s = 0; s < STEPS; ++s) {
         bf16x8 w[QP_NT];
 #pragma unroll
-        for (int t = 0; t < QP_NT; ++t) {
-          if constexpr (WF == QW_I8) {
-            w[t] = scale_bytes_seq<ACT>(cw[t][2 * s] ^ 0x80808080u, cw[t][2 * s + 1] ^ 0x80808080u, s4[t][s],
-                                        -128.0f * s4[t][s]);
-          } else {
-            const uint32_t r = cw[t][s];
-            w[t] = scale_bytes<ACT>(r & 0x0f0f0f0fu, (r >> 4) & 0x0f0f0f0fu, s4[t][s], -8.0f * s4[t][s]);
-          }
-        }
+        for (int t = 0; t < QP_NT; ++t) w[t] = weight_operand<ACT, WF, DW>(cw[t], s, s4[t][s]);
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
           const bf16x8 xr = read_a(i, s);
@@ -393,6 +407,153 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
   }
 }
 
+// A few rows against one quantised matrix: 16 SUB rows by 64 weight rows per
+// workgroup, its four waves taking every fourth K slice each, with codes and
+// activation operands straight in registers one slice ahead, no LDS ring and no
+// barrier in the K loop; the four partial tiles are added in wave order.
+// Bound by the latency of a wave's chain of slices: with 256 weight rows per
+// workgroup (the kernel above) 2048 x 7168 gives 28 workgroups of 16 or 32
+// slices each, 24 to 34 us; here 112 workgroups of 4 or 8 slices per wave, 12
+// us, which is the caller's own time per call (225 us on the general kernel).
+template <int ACT, int WF, int SUB, int KS, bool RS>
+__global__ __launch_bounds__(QP_THREADS, 2) void quant_split_kernel(const uint16_t* __restrict__ x, int rows,
+                                                                    const MfW w, int n_w, int K,
+                                                                    uint16_t* __restrict__ out, int n_tiles,
+                                                                    int chunks) {
+  constexpr int STEPS = KS / 32, DW = qp_dwords<WF, KS>();
+  constexpr int ROWS = 16 * SUB, COLS = 16 * QP_NT;
+  __shared__ __attribute__((aligned(16))) float part[4][ROWS * COLS];
+  // the row chunks of a column tile on one XCD: its weights are fetched by one L2
+  const int b = blockIdx.x, xcd = b % kXcds, j = b / kXcds;
+  const int nt = j / chunks * kXcds + xcd, r0 = j % chunks * ROWS;
+  if (nt >= n_tiles) return;
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int l16 = lane % 16, lq = lane / 16;
+  const int n0 = nt * COLS, KT = K / KS;
+  const int piece = (WF == QW_U4 && KS == 128) ? lq : ((lq & 1) << 1 | (lq >> 1));
+  const char* b_src[QP_NT];
+  const float* s_src[QP_NT];
+  float row_sc[QP_NT];
+#pragma unroll
+  for (int t = 0; t < QP_NT; ++t) {
+    const int wrow = min(n0 + 16 * t + l16, n_w - 1);
+    b_src[t] = w.w + wrow * w.row_bytes + piece * (4 * DW);
+    s_src[t] = w.scales + static_cast<int64_t>(wrow) * w.groups;
+    row_sc[t] = RS ? s_src[t][0] : 0.0f;
+  }
+  const uint16_t* a_src[SUB];
+#pragma unroll
+  for (int i = 0; i < SUB; ++i) a_src[i] = x + static_cast<int64_t>(min(r0 + 16 * i + l16, rows - 1)) * K + 8 * lq;
+  const int step32 = KS == 128 ? lq : (lq & 1), group32 = w.group / 32;
+
+  uint32_t raw[2][QP_NT][DW];
+  float sc[2][QP_NT];
+  bf16x8 xa[2][SUB][STEPS];
+  auto load = [&](int kt, auto buf) {
+    constexpr int B = decltype(buf)::value;
+#pragma unroll
+    for (int t = 0; t < QP_NT; ++t) load_codes<DW>(b_src[t] + kt * (16 * DW), raw[B][t]);
+    if constexpr (!RS) {
+      const int step = kt * STEPS + step32;
+      const int idx = group32 == 1 ? step : step / group32;
+#pragma unroll
+      for (int t = 0; t < QP_NT; ++t) sc[B][t] = s_src[t][idx];
+    }
+#pragma unroll
+    for (int i = 0; i < SUB; ++i)
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) xa[B][i][s] = *reinterpret_cast<const bf16x8*>(a_src[i] + kt * KS + 32 * s);
+  };
+  f32x4 acc[SUB][QP_NT];
+#pragma unroll
+  for (int i = 0; i < SUB; ++i)
+#pragma unroll
+    for (int t = 0; t < QP_NT; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto slice = [&](int kt, auto buf) {
+    constexpr int B = decltype(buf)::value;
+    load(min(kt + 4, KT - 1), std::integral_constant<int, 1 - B>{});  // past the end: the last slice again, unused
+    uint32_t cw[QP_NT][DW];
+    float cs[QP_NT], s4[QP_NT][STEPS];
+#pragma unroll
+    for (int t = 0; t < QP_NT; ++t) {
+#pragma unroll
+      for (int i = 0; i < DW; ++i) cw[t][i] = raw[B][t][i];
+      cs[t] = RS ? row_sc[t] : sc[B][t];
+    }
+    exchange<WF, KS, RS>(cw, cs, s4);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int t = 0; t < QP_NT; ++t) {
+        const bf16x8 f = weight_operand<ACT, WF, DW>(cw[t], s, s4[t][s]);
+#pragma unroll
+        for (int i = 0; i < SUB; ++i) acc[i][t] = mfma_step<ACT>(f, xa[B][i][s], acc[i][t]);
+      }
+  };
+  if (wave < KT) {
+    load(wave, std::integral_constant<int, 0>{});
+    for (int kt = wave; kt < KT; kt += 8) {
+      slice(kt, std::integral_constant<int, 0>{});
+      if (kt + 4 < KT) slice(kt + 4, std::integral_constant<int, 1>{});
+    }
+  }
+  // a lane holds row l16, columns 4 lq .. + 3 of each tile: 16-byte chunk c of
+  // row r at chunk c ^ (r & 15), so the 16 rows of a quarter hit all banks
+#pragma unroll
+  for (int i = 0; i < SUB; ++i)
+#pragma unroll
+    for (int t = 0; t < QP_NT; ++t) {
+      const int r = 16 * i + l16, c = 4 * t + lq;
+      *reinterpret_cast<f32x4*>(&part[wave][r * COLS + 4 * (c ^ l16)]) = acc[i][t];
+    }
+  __syncthreads();
+  const bool vec = n_w % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
+#pragma unroll
+  for (int u = 0; u < ROWS * COLS / 4 / QP_THREADS; ++u) {
+    const int at = tid + u * QP_THREADS, r = at / (COLS / 4), c = at % (COLS / 4);
+    const int col = n0 + 4 * c, row = r0 + r;
+    if (row >= rows || col >= n_w) continue;
+    f32x4 v = *reinterpret_cast<const f32x4*>(&part[0][r * COLS + 4 * (c ^ (r & 15))]);
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v += *reinterpret_cast<const f32x4*>(&part[q][r * COLS + 4 * (c ^ (r & 15))]);
+    uint16_t* o = out + static_cast<int64_t>(row) * n_w + col;
+    if (vec) {
+      *reinterpret_cast<uint2*>(o) = make_uint2(pack_half2<ACT>(v[0], v[1]), pack_half2<ACT>(v[2], v[3]));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (col + k < n_w) o[k] = f32_to_half<ACT>(v[k]);
+    }
+  }
+}
+
+template <int ACT, int WF, int SUB, int KS, bool RS>
+int launch_split(const void* x, int64_t rows, const MfW& w, int64_t n_w, int64_t K, void* out, hipStream_t stream) {
+  const int64_t n_tiles = ceil_div(n_w, 16 * QP_NT), chunks = ceil_div(rows, 16 * SUB);
+  const int64_t grid = kXcds * ceil_div(n_tiles, kXcds) * chunks;
+  if (grid > INT32_MAX) return set_error(QW_ERR_UNSUPPORTED, "quantised matrix grid too large");
+  quant_split_kernel<ACT, WF, SUB, KS, RS><<<static_cast<unsigned>(grid), QP_THREADS, 0, stream>>>(
+      static_cast<const uint16_t*>(x), static_cast<int>(rows), w, static_cast<int>(n_w), static_cast<int>(K),
+      static_cast<uint16_t*>(out), static_cast<int>(n_tiles), static_cast<int>(chunks));
+  QW_LAUNCH_CHECK("quant_split_kernel");
+  return QW_OK;
+}
+
+template <int ACT, int WF>
+int split_any(const void* x, int64_t rows, const MfW& w, int64_t n_w, int64_t K, void* out, hipStream_t stream) {
+  auto go = [&](auto ks, auto rs) -> int {
+    constexpr int KS = decltype(ks)::value;
+    constexpr bool RS = decltype(rs)::value;
+    return rows <= 16 ? launch_split<ACT, WF, 1, KS, RS>(x, rows, w, n_w, K, out, stream)
+                      : launch_split<ACT, WF, 2, KS, RS>(x, rows, w, n_w, K, out, stream);
+  };
+  using K64 = std::integral_constant<int, 64>;
+  if constexpr (WF == QW_U4)
+    return K % 128 == 0 ? go(std::integral_constant<int, 128>{}, std::false_type{}) : go(K64{}, std::false_type{});
+  else
+    return w.groups == 1 ? go(K64{}, std::true_type{}) : go(K64{}, std::false_type{});
+}
+
 struct QpArgs {
   const void* x;
   const int32_t* row_index;
@@ -508,6 +669,19 @@ int quant_matmul(const void* x, int act, const WView& w, int wfmt, int64_t E, co
                  int64_t row_cap, void* out, hipStream_t stream, bool* handled) {
   *handled = false;
   if (!is_half(act) || !quant_fits(w, wfmt) || reinterpret_cast<uintptr_t>(x) % 16 != 0) return QW_OK;
+  // One matrix: the split kernel until its grid is 3.5 workgroups per compute
+  // unit, from where its weights are dequantised too often (int4 2048 x 7168,
+  // split against not: 12 / 34 us at 64 rows, 20 / 35 at 128, 37 / 35 at 256 =
+  // 896 workgroups; 4096 x 1408: 49 / 65 us at 1023 = 704, 97 / 67 at 2048).
+  if (offsets == nullptr && ceil_div(w.rows, 16 * QP_NT) * ceil_div(rows, rows <= 16 ? 16 : 32) <= 896) {
+    const MfW m = mf_view(wfmt, w);
+    const int st = act == QW_F16 ? (wfmt == QW_I8 ? split_any<QW_F16, QW_I8>(x, rows, m, w.rows, w.cols, out, stream)
+                                                  : split_any<QW_F16, QW_U4>(x, rows, m, w.rows, w.cols, out, stream))
+                                 : (wfmt == QW_I8 ? split_any<QW_BF16, QW_I8>(x, rows, m, w.rows, w.cols, out, stream)
+                                                  : split_any<QW_BF16, QW_U4>(x, rows, m, w.rows, w.cols, out, stream));
+    if (st == QW_OK) *handled = true;
+    return st;
+  }
   int sub = pick_sub(E > 1 ? std::min(row_cap, 2 * ceil_div(rows, E)) : rows);
   // a few matrices leave compute units idle in large chunks: smaller ones
   // while there are fewer than two workgroups per unit

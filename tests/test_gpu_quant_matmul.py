@@ -15,8 +15,8 @@ ULP = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}  # of a value in [1
 
 def check(got, x, deq):
     """|error| of each output: half an ulp of the output, half an ulp of every
-    weight (rounded to the activation type by the matrix-core kernels, exact in
-    the streaming ones) times |x|, and the fp32 sum's roundings."""
+    weight (rounded to the activation type) times |x|, and the fp32 sum's
+    roundings."""
     xd = x.double()
     ref = xd @ deq.double().t()
     mass = xd.abs() @ deq.double().abs().t()
