@@ -186,8 +186,8 @@ constexpr int GV_GPW_MAX = 8;  // groups per wave, at most
 template <int WF, int UNITS, int ROWS, int CPL, int MAXM, bool SAVE = false>
 struct GvLds {
   static constexpr int NCH = UNITS * ROWS * CPL;                 // chunk loads per group
-  static_assert(NCH == 4 || NCH == 8, "the ring reads four or eight chunks per group");
   static constexpr bool QUANT = quantized(WF);
+  static_assert(NCH == 4 || NCH == 8 || (NCH == 16 && !QUANT), "the ring reads four, eight or sixteen chunks per group");
   static constexpr int STAGE = NCH * 1024 + (QUANT ? NCH * 256 : 0);
   static constexpr int STAGES = 2;
   static constexpr int NDMA = NCH * (QUANT ? 2 : 1);             // DMA instructions per group
@@ -582,7 +582,18 @@ __global__ __launch_bounds__(GV_WAVES * 64) void ffn_gemv_kernel(
       const char* st = ring + ((g - g_first) % LD::STAGES) * LD::STAGE;
       uint4 wq[LD::NCH];
       float sq[LD::NCH];
-      if constexpr (LD::NCH == 8)
+      if constexpr (LD::NCH == 16) {
+        uint4 lo[8], hi[8];
+        float none[8];
+        ring_read8<false>(lds_addr(st) + lane * 16, 0u, lo, none);
+        ring_read8<false>(lds_addr(st) + 8192 + lane * 16, 0u, hi, none);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          wq[i] = lo[i];
+          wq[8 + i] = hi[i];
+          sq[i] = sq[8 + i] = 1.0f;
+        }
+      } else if constexpr (LD::NCH == 8)
         ring_read8<LD::QUANT>(lds_addr(st) + lane * 16, lds_addr(st + LD::NCH * 1024) + lane * 4, wq, sq);
       else
         ring_read4<LD::QUANT>(lds_addr(st) + lane * 16, lds_addr(st + LD::NCH * 1024) + lane * 4, wq, sq);
@@ -1304,7 +1315,9 @@ int launch_qmf(const FfnArgs& a, const WView& wa, const WView& wb, const void* x
 }
 
 // Units per group for a row of CPL chunks per lane: 4 weight chunks (16-byte
-// loads) per lane and group (8 for gate/up rows of more than 128 chunks).
+// loads) per lane and group (8 for gate/up rows of more than 128 chunks, 16 for
+// 16-bit gate/up rows of more than 256: bf16 d 4096 took the general kernel
+// before, 741 us for one token's layer call against 39).
 template <int ACT, int WF, bool GATEUP>
 int launch_cpl(const FfnArgs& a, const WView& wa, const WView& wb, const void* x, const int32_t* row_index, int K,
                int n_out, const float* row_weight, void* out, void* save_a, void* save_b, hipStream_t stream) {
@@ -1318,6 +1331,10 @@ int launch_cpl(const FfnArgs& a, const WView& wa, const WView& wb, const void* x
                                              stream);
   if (cpl <= 4)
     return launch_one<ACT, WF, GATEUP, 1, 4>(a, wa, wb, x, row_index, K, n_out, row_weight, out, save_a, save_b, stream);
+  if constexpr (!quantized(WF))
+    if (cpl <= 8)
+      return launch_one<ACT, WF, GATEUP, 1, 8>(a, wa, wb, x, row_index, K, n_out, row_weight, out, save_a, save_b,
+                                               stream);
   return set_error(QW_ERR_UNSUPPORTED, "row of %d chunks is too long for the decode kernel", KC);
 }
 
@@ -1348,7 +1365,14 @@ int launch_fmt(const FfnArgs& a, hipStream_t stream) {
 
 int launch_ffn_gemv(const FfnArgs& a, hipStream_t stream, bool* handled) {
   *handled = false;
-  if (!is_half(a.act) || a.avg_rows >= 16) return QW_OK;
+  // 16-bit weights: a pass takes 4 rows of an expert and reads all its weights,
+  // the matrix-core kernel reads them once whatever the rows (whole layer, 64
+  // experts, d 2048, f 1024, streamed against not: 70 / 95 us at 16 tokens, 135
+  // / 137 at 64 = 2 rows per expert, 180 / 150 at 96, 206 / 153 at 128, 405 /
+  // 159 at 333).  Quantised weights: the streaming kernels multiply the exact
+  // codes, the matrix-core ones rounded weights, and take over only where they
+  // always did.
+  if (!is_half(a.act) || a.avg_rows >= (quantized(a.wfmt) ? 16 : 3)) return QW_OK;
   const bool f16 = a.act == QW_F16;
   if ((a.save_gate || a.save_y) && quantized(a.wfmt)) return QW_OK;  // quantised experts do not train
   // the matrix-core decode kernel's grid has a row per pass of up to 4 routes:
@@ -1368,7 +1392,8 @@ int launch_ffn_gemv(const FfnArgs& a, hipStream_t stream, bool* handled) {
     return QW_OK;
   }
   if (a.d_model % cw || a.d_ff % cw) return QW_OK;
-  if (ceil_div(a.d_model / cw, 64) > 4 || ceil_div(a.d_ff / cw, 64) > 4) return QW_OK;
+  const int most = quantized(a.wfmt) ? 4 : 8;  // chunks per lane the kernels take
+  if (ceil_div(a.d_model / cw, 64) > most || ceil_div(a.d_ff / cw, 64) > most) return QW_OK;
   // the padded int4/int8 row must equal the logical row (true when K is a multiple of the group)
   if (quantized(a.wfmt) && (a.gate.row_stride * (a.wfmt == QW_U4 ? 2 : 1) != a.d_model ||
                             a.down.row_stride * (a.wfmt == QW_U4 ? 2 : 1) != a.d_ff))

@@ -579,10 +579,12 @@ int launch_ffn_mfma(const FfnArgs& a, hipStream_t stream, bool* handled) {
   if (quant && likely_rows(a, 2.0) <= kQuantRows) return QW_OK;  // dequantised once per weight instead of twice
   // An expert's second chunk reads all its weights again and, started last,
   // costs a whole workgroup's time (T = 7000, capacity 274: 292 us in chunks
-  // of 256 rows against 248 us in chunks of 320): the bound where one chunk
-  // holds it, else room for 3.5 standard deviations (T = 512 without capacity:
-  // 163 us in chunks of 64 rows against 181 us in chunks of 320).
-  const int subt = pick_subt(rows_cap <= 320 ? rows_cap : likely_rows(a, 3.5));
+  // of 256 rows against 248 us in chunks of 320): a capacity bound decides where
+  // one chunk holds it.  A bound far above the average (no capacity) would only
+  // widen the activation slices of nearly empty chunks (T = 512: 181 us in
+  // chunks of 320 rows, 163 us in chunks of 64): room for 3.5 standard deviations.
+  const bool bound = rows_cap <= 320 && rows_cap <= 2 * a.avg_rows;
+  const int subt = pick_subt(bound ? rows_cap : likely_rows(a, 3.5));
   const int D = static_cast<int>(a.d_model), F = static_cast<int>(a.d_ff), E = static_cast<int>(a.experts);
   const int mr = static_cast<int>(a.max_rows);
   const MfW g = mf_view(a.wfmt, a.gate), u = mf_view(a.wfmt, a.up), dn = mf_view(a.wfmt, a.down);
