@@ -214,6 +214,22 @@ int qw_moe_forward(const void* x, int act_dtype, int64_t tokens, int64_t d_model
                    int32_t* totals, int32_t* dropped_token, int32_t* dropped_expert, void* workspace,
                    size_t workspace_bytes, void* stream);
 
+/* qw_moe_forward that also returns what TopKMoE.forward computes beside the
+ * output: importance [experts] and the balance loss of qw_moe_balance_ws (same
+ * additions in the same order), the dropped-route count as a 64-bit integer,
+ * and a zero (the domain loss when none is asked for).  They ride on the plan
+ * and combine launches. */
+size_t qw_moe_forward_balance_workspace_bytes(int64_t tokens, int64_t d_model, int64_t experts, int64_t top_k,
+                                              int64_t d_ff, int act_dtype);
+int qw_moe_forward_balance(const void* x, int act_dtype, int64_t tokens, int64_t d_model, const void* router_w,
+                   int router_dtype, float temperature, const float* expert_bias, int64_t experts, int64_t top_k,
+                   int64_t capacity, int64_t d_ff, int w_format, int64_t group_in, int64_t group_ff,
+                   const void* gate_w, const float* gate_scales, const void* up_w, const float* up_scales,
+                   const void* down_w, const float* down_scales, void* out, float* probs, int32_t* top_idx,
+                   float* top_w, int32_t* counts, int32_t* kept_counts, int32_t* totals, int32_t* dropped_token,
+                   int32_t* dropped_expert, float* importance, float* balance_out, int64_t* overflow_out,
+                           float* zero_out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* One decode step of a MoE layer, the routed-expert lines of
  * FastDecoder._step (src/fast_decode.py:170-177), with the experts kept in
  * their stored format (the reference stacks dense dequantised copies,

@@ -42,6 +42,9 @@ SIGNATURES = {
     "qw_moe_forward_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I32]),
     "qw_moe_forward": (I32, [P, I32, I64, I64, P, I32, F32, P, I64, I64, I64, I64, I32, I64, I64,
                              P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, SZ, P]),
+    "qw_moe_forward_balance_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I32]),
+    "qw_moe_forward_balance": (I32, [P, I32, I64, I64, P, I32, F32, P, I64, I64, I64, I64, I32, I64, I64,
+                                     P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, SZ, P]),
     "qw_moe_decode_step_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I32]),
     "qw_moe_decode_step": (I32, [P, P, I64, I64, P, F32, P, I64, I64, I64, I32, I32, I64, I64,
                                  P, P, P, P, P, P, P, P, P, P, P, SZ, P]),

@@ -7,6 +7,7 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "qw_balance.h"
 #include "qw_ffn.h"
 
 namespace qw {
@@ -42,7 +43,7 @@ int route_plan_small(const void* x, int xdt, int64_t x_stride, const void* w, in
 int plan(const int32_t* top_idx, const float* top_w, int64_t T, int64_t K, int64_t E, int64_t capacity,
          int32_t* counts, int32_t* kept_counts, int32_t* kept_offsets, int32_t* slot_token, float* slot_weight,
          int32_t* route_slot, int32_t* dropped_token, int32_t* dropped_expert, int32_t* totals, void* ws,
-         size_t ws_bytes, hipStream_t stream);
+         size_t ws_bytes, hipStream_t stream, const BalanceJob& job = BalanceJob());
 int permute(const void* x, int dtype, int64_t D, const int32_t* slot_token, const int32_t* totals, int64_t max_rows,
             void* out, hipStream_t stream);
 int combine(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, int64_t T, int64_t K,
@@ -64,6 +65,9 @@ int grouped_matmul_generic(const void* x, int act, const WView& w, int wfmt, int
                            int64_t rows, void* out, hipStream_t stream);
 int combine_weighted(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
                      int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream);
+int combine_balance(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
+                    int64_t T, int64_t K, int64_t D, void* out, int out_dtype, const BalanceJob& job,
+                    hipStream_t stream);
 int combine_static(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
                    int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream);
 int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
@@ -268,6 +272,72 @@ static int current_device(int* dev) {
   return QW_OK;
 }
 
+// The layer forward; with job.balance also its balance loss, as extra
+// workgroups of the plan and combine launches.
+static int layer_forward(const void* x, int act_dtype, int64_t tokens, int64_t d_model, const void* router_w,
+                   int router_dtype, float temperature, const float* expert_bias, int64_t experts, int64_t top_k,
+                   int64_t capacity, int64_t d_ff, int w_format, int64_t group_in, int64_t group_ff,
+                   const void* gate_w, const float* gate_scales, const void* up_w, const float* up_scales,
+                   const void* down_w, const float* down_scales, void* out, float* probs, int32_t* top_idx,
+                   float* top_w, int32_t* counts, int32_t* kept_counts, int32_t* totals, int32_t* dropped_token,
+                   int32_t* dropped_expert, void* workspace, size_t workspace_bytes, hipStream_t s,
+                   const BalanceJob& job) {
+  QW_REQUIRE(act_dtype == QW_F32 || act_dtype == QW_BF16 || act_dtype == QW_F16,
+             "activation dtype must be f32, bf16 or f16");
+  QW_REQUIRE(tokens >= 0 && top_k >= 1 && experts >= 1 && d_model >= 1 && d_ff >= 1, "bad forward sizes");
+  QW_REQUIRE(capacity >= 0, "capacity must be >= 0");
+  QW_REQUIRE(probs && top_idx && top_w && counts && kept_counts && totals, "forward outputs are required");
+  if (tokens == 0) return QW_OK;
+  QW_REQUIRE(out && dropped_token && dropped_expert, "forward outputs are required");
+  const size_t need = forward_workspace_bytes(tokens, d_model, experts, top_k, d_ff, act_dtype);
+  if (!workspace || workspace_bytes < need)
+    return set_error(QW_ERR_WORKSPACE, "forward workspace needs %zu bytes, got %zu", need, workspace_bytes);
+  const int64_t R = tokens * top_k;
+  Carver c(workspace);
+  float* logits = c.take<float>(static_cast<size_t>(tokens) * experts);
+  int32_t* slot_token = c.take<int32_t>(R);
+  float* slot_weight = c.take<float>(R);
+  int32_t* route_slot = c.take<int32_t>(R);
+  int32_t* kept_offsets = c.take<int32_t>(experts + 1);
+  char* y = c.take<char>(static_cast<size_t>(R) * d_model * act_size(act_dtype));
+  const size_t plan_ws = plan_workspace_bytes(tokens, top_k, experts);
+  char* pws = c.take<char>(plan_ws);
+  const int64_t max_rows = std::min<int64_t>(R, capacity * experts);
+  const size_t exp_ws = experts_workspace_bytes(R, experts, d_model, d_ff, act_dtype);
+  char* ews = c.take<char>(exp_ws);
+  const size_t route_ws = route_workspace_bytes(tokens, d_model, experts);
+  float* rws = reinterpret_cast<float*>(c.take<char>(route_ws));
+  int st;
+  if (route_plan_small_fits(tokens, experts, top_k)) {
+    st = route_plan_small(x, act_dtype, d_model, router_w, router_dtype, tokens, d_model, experts, top_k, temperature,
+                          expert_bias, false, logits, probs, top_idx, top_w, capacity, counts, kept_counts,
+                          kept_offsets, totals, slot_token, slot_weight, route_slot, dropped_token, dropped_expert,
+                          nullptr, nullptr, act_dtype, rws, route_ws, s);
+    if (st) return st;
+  } else {
+    st = route(x, act_dtype, d_model, router_w, router_dtype, tokens, d_model, experts, top_k, temperature,
+               expert_bias, logits, probs, top_idx, top_w, rws, route_ws, s);
+    if (st) return st;
+    st = plan(top_idx, top_w, tokens, top_k, experts, capacity, counts, kept_counts, kept_offsets, slot_token,
+              slot_weight, route_slot, dropped_token, dropped_expert, totals, pws, plan_ws, s, job);
+    if (st) return st;
+  }
+  // The experts store unweighted rows and the combine applies the route
+  // weights: it computes the same bf16(bf16(y) * w) per route that the
+  // expert kernels would store, and the down projection's epilogue then waits
+  // on no weight loads.
+  if (max_rows > 0) {
+    const int64_t avg = (R + experts - 1) / experts;
+    st = qw::experts(x, act_dtype, slot_token, kept_offsets, experts, d_model, d_ff, max_rows, w_format, group_in,
+                     group_ff, gate_w, gate_scales, up_w, up_scales, down_w, down_scales, nullptr, y, ews, exp_ws, s,
+                     avg < capacity ? avg : capacity, std::min<int64_t>(capacity, R));
+    if (st) return st;
+  }
+  if (job.balance != nullptr)
+    return combine_balance(y, act_dtype, route_slot, top_idx, top_w, tokens, top_k, d_model, out, act_dtype, job, s);
+  return combine_weighted(y, act_dtype, route_slot, top_idx, top_w, tokens, top_k, d_model, out, act_dtype, s);
+}
+
 }  // namespace qw
 
 using namespace qw;
@@ -418,59 +488,53 @@ int qw_moe_forward(const void* x, int act_dtype, int64_t tokens, int64_t d_model
                    float* top_w, int32_t* counts, int32_t* kept_counts, int32_t* totals, int32_t* dropped_token,
                    int32_t* dropped_expert, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
-  QW_REQUIRE(act_dtype == QW_F32 || act_dtype == QW_BF16 || act_dtype == QW_F16,
-             "activation dtype must be f32, bf16 or f16");
+  return layer_forward(x, act_dtype, tokens, d_model, router_w, router_dtype, temperature, expert_bias, experts, top_k,
+                 capacity, d_ff, w_format, group_in, group_ff, gate_w, gate_scales, up_w, up_scales, down_w,
+                 down_scales, out, probs, top_idx, top_w, counts, kept_counts, totals, dropped_token,
+                 dropped_expert, workspace, workspace_bytes, as_stream(stream), BalanceJob());
+}
+
+size_t qw_moe_forward_balance_workspace_bytes(int64_t tokens, int64_t d_model, int64_t experts, int64_t top_k,
+                                              int64_t d_ff, int act_dtype) {
+  if (tokens < 0 || d_model < 1 || experts < 1 || top_k < 1 || d_ff < 1) return 0;
+  return align_up(forward_workspace_bytes(tokens, d_model, experts, top_k, d_ff, act_dtype), 256) +
+         balance_workspace_bytes(tokens, experts);
+}
+
+int qw_moe_forward_balance(const void* x, int act_dtype, int64_t tokens, int64_t d_model, const void* router_w,
+                   int router_dtype, float temperature, const float* expert_bias, int64_t experts, int64_t top_k,
+                   int64_t capacity, int64_t d_ff, int w_format, int64_t group_in, int64_t group_ff,
+                   const void* gate_w, const float* gate_scales, const void* up_w, const float* up_scales,
+                   const void* down_w, const float* down_scales, void* out, float* probs, int32_t* top_idx,
+                   float* top_w, int32_t* counts, int32_t* kept_counts, int32_t* totals, int32_t* dropped_token,
+                   int32_t* dropped_expert, float* importance, float* balance_out, int64_t* overflow_out,
+                           float* zero_out, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
   QW_REQUIRE(tokens >= 0 && top_k >= 1 && experts >= 1 && d_model >= 1 && d_ff >= 1, "bad forward sizes");
-  QW_REQUIRE(capacity >= 0, "capacity must be >= 0");
-  QW_REQUIRE(probs && top_idx && top_w && counts && kept_counts && totals, "forward outputs are required");
+  QW_REQUIRE(importance && balance_out && overflow_out && zero_out, "the balance outputs are required");
   if (tokens == 0) return QW_OK;
-  QW_REQUIRE(out && dropped_token && dropped_expert, "forward outputs are required");
-  const size_t need = forward_workspace_bytes(tokens, d_model, experts, top_k, d_ff, act_dtype);
+  QW_REQUIRE(tokens <= INT32_MAX && experts <= 1024, "bad balance sizes");
+  const size_t need = qw_moe_forward_balance_workspace_bytes(tokens, d_model, experts, top_k, d_ff, act_dtype);
   if (!workspace || workspace_bytes < need)
     return set_error(QW_ERR_WORKSPACE, "forward workspace needs %zu bytes, got %zu", need, workspace_bytes);
-  hipStream_t s = as_stream(stream);
-  const int64_t R = tokens * top_k;
-  Carver c(workspace);
-  float* logits = c.take<float>(static_cast<size_t>(tokens) * experts);
-  int32_t* slot_token = c.take<int32_t>(R);
-  float* slot_weight = c.take<float>(R);
-  int32_t* route_slot = c.take<int32_t>(R);
-  int32_t* kept_offsets = c.take<int32_t>(experts + 1);
-  char* y = c.take<char>(static_cast<size_t>(R) * d_model * act_size(act_dtype));
-  const size_t plan_ws = plan_workspace_bytes(tokens, top_k, experts);
-  char* pws = c.take<char>(plan_ws);
-  const int64_t max_rows = std::min<int64_t>(R, capacity * experts);
-  const size_t exp_ws = experts_workspace_bytes(R, experts, d_model, d_ff, act_dtype);
-  char* ews = c.take<char>(exp_ws);
-  const size_t route_ws = route_workspace_bytes(tokens, d_model, experts);
-  float* rws = reinterpret_cast<float*>(c.take<char>(route_ws));
-  int st;
-  if (route_plan_small_fits(tokens, experts, top_k)) {
-    st = route_plan_small(x, act_dtype, d_model, router_w, router_dtype, tokens, d_model, experts, top_k, temperature,
-                          expert_bias, false, logits, probs, top_idx, top_w, capacity, counts, kept_counts,
-                          kept_offsets, totals, slot_token, slot_weight, route_slot, dropped_token, dropped_expert,
-                          nullptr, nullptr, act_dtype, rws, route_ws, s);
-    if (st) return st;
-  } else {
-    st = route(x, act_dtype, d_model, router_w, router_dtype, tokens, d_model, experts, top_k, temperature,
-               expert_bias, logits, probs, top_idx, top_w, rws, route_ws, s);
-    if (st) return st;
-    st = plan(top_idx, top_w, tokens, top_k, experts, capacity, counts, kept_counts, kept_offsets, slot_token,
-              slot_weight, route_slot, dropped_token, dropped_expert, totals, pws, plan_ws, s);
-    if (st) return st;
-  }
-  // The experts store unweighted rows and the combine applies the route
-  // weights: it computes the same bf16(bf16(y) * w) per route that the
-  // expert kernels would store, and the down projection's epilogue then waits
-  // on no weight loads.
-  if (max_rows > 0) {
-    const int64_t avg = (R + experts - 1) / experts;
-    st = qw::experts(x, act_dtype, slot_token, kept_offsets, experts, d_model, d_ff, max_rows, w_format, group_in,
-                     group_ff, gate_w, gate_scales, up_w, up_scales, down_w, down_scales, nullptr, y, ews, exp_ws, s,
-                     avg < capacity ? avg : capacity, std::min<int64_t>(capacity, R));
-    if (st) return st;
-  }
-  return combine_weighted(y, act_dtype, route_slot, top_idx, top_w, tokens, top_k, d_model, out, act_dtype, s);
+  const size_t used = align_up(forward_workspace_bytes(tokens, d_model, experts, top_k, d_ff, act_dtype), 256);
+  BalanceJob job;
+  job.probs = probs;
+  job.counts = counts;
+  job.totals = totals;
+  job.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + used);
+  job.nb = static_cast<int>(ceil_div(tokens, kImpRows));
+  job.T = static_cast<int>(tokens);
+  job.K = static_cast<int>(top_k);
+  job.E = static_cast<int>(experts);
+  job.importance = importance;
+  job.balance = balance_out;
+  job.overflow = overflow_out;
+  job.zero = zero_out;
+  return layer_forward(x, act_dtype, tokens, d_model, router_w, router_dtype, temperature, expert_bias, experts, top_k,
+                 capacity, d_ff, w_format, group_in, group_ff, gate_w, gate_scales, up_w, up_scales, down_w,
+                 down_scales, out, probs, top_idx, top_w, counts, kept_counts, totals, dropped_token,
+                 dropped_expert, workspace, used, as_stream(stream), job);
 }
 
 size_t qw_moe_decode_step_workspace_bytes(int64_t tokens, int64_t d_model, int64_t experts, int64_t top_k,

@@ -1,7 +1,8 @@
 // Permute, combine, balance loss, weight quantisation and the plain grouped
 // matmul.
-#include "qw_weights.h"
+#include "qw_balance.h"
 #include "qw_ffn.h"
+#include "qw_weights.h"
 
 namespace qw {
 
@@ -65,12 +66,20 @@ template <int ACT, int OUT, int VEC, int KMAX, bool WEIGHTED, bool STATIC = fals
 __global__ __launch_bounds__(256) void combine_kernel(const void* __restrict__ y, const int32_t* __restrict__ route_slot,
                                                       const int32_t* __restrict__ top_idx,
                                                       const float* __restrict__ top_w, int K, int D,
-                                                      void* __restrict__ out) {
+                                                      void* __restrict__ out, const BalanceJob job) {
   // products and sums rounded one by one (no fused multiply-add): the weighted
   // term is the reference's y * w, rounded to the output dtype before its
   // index_add; the sum is rounded when it is stored
 #pragma clang fp contract(off)
-  const int t = blockIdx.x;
+  if constexpr (WEIGHTED && !STATIC) {  // the first workgroup finishes the balance loss, where it is asked for
+    __shared__ float red[16][kWave];
+    __shared__ float term[1024];
+    if (job.balance != nullptr && blockIdx.x == 0) {
+      balance_final(job, red, term);
+      return;
+    }
+  }
+  const int t = blockIdx.x - (WEIGHTED && !STATIC && job.balance != nullptr ? 1 : 0);
   int sl[KMAX], ex[KMAX];
   float wt[KMAX];
 #pragma unroll
@@ -155,22 +164,22 @@ __global__ __launch_bounds__(256) void combine_kernel(const void* __restrict__ y
 
 template <int ACT, int OUT, int KMAX, bool WEIGHTED, bool STATIC>
 void launch_combine_vec(const void* y, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
-                        unsigned g, int k, int d, void* out, hipStream_t stream) {
+                        unsigned g, int k, int d, void* out, const BalanceJob& job, hipStream_t stream) {
   constexpr int V = (ACT != QW_F32 || OUT != QW_F32) ? 8 : 4;
   if (d % V == 0)
     combine_kernel<ACT, OUT, V, KMAX, WEIGHTED, STATIC>
-        <<<g, 256, 0, stream>>>(y, route_slot, top_idx, top_w, k, d, out);
+        <<<g, 256, 0, stream>>>(y, route_slot, top_idx, top_w, k, d, out, job);
   else
     combine_kernel<ACT, OUT, 1, KMAX, WEIGHTED, STATIC>
-        <<<g, 256, 0, stream>>>(y, route_slot, top_idx, top_w, k, d, out);
+        <<<g, 256, 0, stream>>>(y, route_slot, top_idx, top_w, k, d, out, job);
 }
 
 template <int KMAX, bool WEIGHTED, bool STATIC>
 int launch_combine(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
-                   unsigned g, int k, int d, void* out, int out_dtype, hipStream_t stream) {
+                   unsigned g, int k, int d, void* out, int out_dtype, const BalanceJob& job, hipStream_t stream) {
 #define QW_CB(A, O)                                                                                             \
   if (dtype == A && out_dtype == O)                                                                             \
-    launch_combine_vec<A, O, KMAX, WEIGHTED, STATIC>(y, route_slot, top_idx, top_w, g, k, d, out, stream);   \
+    launch_combine_vec<A, O, KMAX, WEIGHTED, STATIC>(y, route_slot, top_idx, top_w, g, k, d, out, job, stream); \
   else
   QW_CB(QW_F32, QW_F32)
   QW_CB(QW_F32, QW_BF16)
@@ -188,18 +197,19 @@ int launch_combine(const void* y, int dtype, const int32_t* route_slot, const in
 
 template <bool WEIGHTED, bool STATIC = false>
 int combine_k(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
-              int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream) {
-  const unsigned g = static_cast<unsigned>(T);
+              int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream,
+              const BalanceJob& job = BalanceJob()) {
+  const unsigned g = static_cast<unsigned>(T) + (job.balance != nullptr ? 1 : 0);
   const int k = static_cast<int>(K), d = static_cast<int>(D);
 #define QW_CK(N)                                                                                                 \
   if (K <= N)                                                                                                    \
-    return launch_combine<N, WEIGHTED, STATIC>(y, dtype, route_slot, top_idx, top_w, g, k, d, out, out_dtype, stream);
+    return launch_combine<N, WEIGHTED, STATIC>(y, dtype, route_slot, top_idx, top_w, g, k, d, out, out_dtype, job, stream);
   QW_CK(2)
   QW_CK(4)
   QW_CK(8)
   QW_CK(16)
 #undef QW_CK
-  return launch_combine<64, WEIGHTED, STATIC>(y, dtype, route_slot, top_idx, top_w, g, k, d, out, out_dtype, stream);
+  return launch_combine<64, WEIGHTED, STATIC>(y, dtype, route_slot, top_idx, top_w, g, k, d, out, out_dtype, job, stream);
 }
 
 static int combine_check(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, int64_t T,
@@ -221,6 +231,14 @@ int combine_weighted(const void* y, int dtype, const int32_t* route_slot, const 
   if (T == 0) return QW_OK;
   if (top_w) return combine_k<true>(y, dtype, route_slot, top_idx, top_w, T, K, D, out, out_dtype, stream);
   return combine_k<false>(y, dtype, route_slot, top_idx, nullptr, T, K, D, out, out_dtype, stream);
+}
+
+// The weighted combine that also finishes the balance loss of `job`.
+int combine_balance(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
+                    int64_t T, int64_t K, int64_t D, void* out, int out_dtype, const BalanceJob& job,
+                    hipStream_t stream) {
+  if (const int st = combine_check(y, dtype, route_slot, top_idx, T, K, D, out, out_dtype)) return st;
+  return combine_k<true>(y, dtype, route_slot, top_idx, top_w, T, K, D, out, out_dtype, stream, job);
 }
 
 int combine_static(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
@@ -460,87 +478,18 @@ __global__ void balance_kernel(const float* __restrict__ importance, const int32
   *balance = static_cast<float>(E) * s;
 }
 
-// The same with per-workgroup partial sums (coalesced row reads over token
-// chunks) summed afterwards in a fixed order: deterministic, and the probs
-// matrix is read by many CUs instead of one workgroup per strided column.
-constexpr int kImpRows = 64;  // tokens per partial-sum workgroup
-
-__global__ __launch_bounds__(256) void importance_partial_kernel(const float* __restrict__ probs, int T, int E,
-                                                                 float* __restrict__ partial) {
-  __shared__ float red[4][64];
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int e = blockIdx.y * 64 + lane;
-  const int t0 = blockIdx.x * kImpRows, t1 = min(T, t0 + kImpRows);
-  // all of the thread's loads in flight at once, then added in token order
-  // (a token past the end adds +0, which leaves the non-negative sum as it is)
-  float v[kImpRows / 4];
-#pragma unroll
-  for (int i = 0; i < kImpRows / 4; ++i) {
-    const int t = t0 + wave + 4 * i;
-    v[i] = (e < E && t < t1) ? probs[static_cast<int64_t>(t) * E + e] : 0.0f;
-  }
-  float s = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kImpRows / 4; ++i) s += v[i];
-  red[wave][lane] = s;
-  __syncthreads();
-  if (wave == 0 && e < E)
-    partial[static_cast<int64_t>(blockIdx.x) * E + e] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+// The same with partial sums per 64 tokens (coalesced row reads) summed
+// afterwards in a fixed order: deterministic, and the probs matrix is read by
+// many CUs instead of one workgroup per strided column.
+__global__ __launch_bounds__(256) void importance_partial_kernel(const BalanceJob job) {
+  __shared__ float red[4][kWave];
+  importance_unit(job, blockIdx.x, red);
 }
 
-// One workgroup of 16 waves; lane l holds expert e0 + l of each 64-expert
-// block.  Wave w adds the partial rows w, w + 16, ... in order (whole rows:
-// coalesced loads, all of a wave's rows in flight together), the 16 wave sums
-// are added in wave order, so importance[e] = sum / T does not depend on
-// scheduling.  The balance term is then summed over experts in ascending order
-// by one thread.
-__global__ __launch_bounds__(1024) void importance_final_kernel(const float* __restrict__ partial, int nb, int T,
-                                                                int K, int E, const int32_t* __restrict__ counts,
-                                                                float* __restrict__ importance,
-                                                                float* __restrict__ balance) {
-  constexpr int kW = 16, kRowsPerLoad = 8;
+__global__ __launch_bounds__(256) void importance_final_kernel(const BalanceJob job) {
+  __shared__ float red[16][kWave];
   __shared__ float term[1024];
-  __shared__ float red[kW][kWave];
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const float routes = static_cast<float>(static_cast<int64_t>(T) * K);
-  for (int e0 = 0; e0 < E; e0 += kWave) {
-    const int e = e0 + lane;
-    float s = 0.0f;
-    for (int b0 = wave; b0 < nb; b0 += kW * kRowsPerLoad) {
-      float v[kRowsPerLoad];
-#pragma unroll
-      for (int i = 0; i < kRowsPerLoad; ++i) {
-        const int b = b0 + kW * i;
-        v[i] = (b < nb && e < E) ? partial[static_cast<int64_t>(b) * E + e] : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < kRowsPerLoad; ++i) s += v[i];  // rows in order; +0 past the end (sums are >= 0)
-    }
-    red[wave][lane] = s;
-    __syncthreads();
-    if (wave == 0 && e < E) {
-      float t = 0.0f;
-#pragma unroll
-      for (int w = 0; w < kW; ++w) t += red[w][lane];
-      const float imp = t / static_cast<float>(T);
-      importance[e] = imp;
-      term[e] = imp * (static_cast<float>(counts[e]) / routes);
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    // ascending order; 16 reads in flight at a time (the terms are >= 0, so
-    // the +0 past E changes nothing)
-    float s = 0.0f;
-    for (int e0 = 0; e0 < E; e0 += 16) {
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = e0 + i < E ? term[e0 + i] : 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s += v[i];
-    }
-    *balance = static_cast<float>(E) * s;
-  }
+  balance_final(job, red, term);
 }
 
 size_t balance_workspace_bytes(int64_t T, int64_t E) {
@@ -554,13 +503,21 @@ int balance_ws(const float* probs, const int32_t* counts, int64_t T, int64_t K, 
   const size_t need = balance_workspace_bytes(T, E);
   if (!ws || ws_bytes < need)
     return set_error(QW_ERR_WORKSPACE, "balance workspace needs %zu bytes, got %zu", need, ws_bytes);
-  const int nb = static_cast<int>(ceil_div(T, kImpRows));
-  float* partial = static_cast<float*>(ws);
-  const dim3 g(static_cast<unsigned>(nb), static_cast<unsigned>(ceil_div(E, 64)));
-  importance_partial_kernel<<<g, 256, 0, stream>>>(probs, static_cast<int>(T), static_cast<int>(E), partial);
-  QW_LAUNCH_CHECK("importance_partial_kernel");
-  importance_final_kernel<<<1, 1024, 0, stream>>>(partial, nb, static_cast<int>(T), static_cast<int>(K),
-                                                   static_cast<int>(E), counts, importance, bal);
+  BalanceJob job;
+  job.probs = probs;
+  job.counts = counts;
+  job.partial = static_cast<float*>(ws);
+  job.nb = static_cast<int>(ceil_div(T, kImpRows));
+  job.T = static_cast<int>(T);
+  job.K = static_cast<int>(K);
+  job.E = static_cast<int>(E);
+  job.importance = importance;
+  job.balance = bal;
+  if (job.nb > 1) {
+    importance_partial_kernel<<<static_cast<unsigned>(partial_units(job.nb, job.E)), 256, 0, stream>>>(job);
+    QW_LAUNCH_CHECK("importance_partial_kernel");
+  }
+  importance_final_kernel<<<1, 256, 0, stream>>>(job);
   QW_LAUNCH_CHECK("importance_final_kernel");
   return QW_OK;
 }

@@ -23,7 +23,7 @@
 // holds gathers its keys into its own slice of the workspace and sorts them
 // there with a bitonic network (same result, slower: one global-memory pass
 // per network stage).
-#include "qw_common.h"
+#include "qw_balance.h"
 
 namespace qw {
 
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
     int32_t* __restrict__ counts, int32_t* __restrict__ kept_counts, int32_t* __restrict__ kept_offsets,
     int32_t* __restrict__ totals, int32_t* __restrict__ slot_token, float* __restrict__ slot_weight,
     int32_t* __restrict__ route_slot, int32_t* __restrict__ dropped_token, int32_t* __restrict__ dropped_expert,
-    uint64_t* __restrict__ spill) {
+    uint64_t* __restrict__ spill, const BalanceJob job) {
   constexpr int kWaves = kPlanThreads / kWave;
   // Two key buffers; the second holds the per-wave histograms until the
   // offsets are known.
@@ -123,6 +123,11 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(
   __shared__ int s_kept_off, s_drop_off, s_route_off, s_fill, s_fill_big;
   const int e = blockIdx.x;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  if (e >= E) {  // workgroups past the experts: the balance loss's partial sums, one unit per four waves
+    float (*const red)[kWave] = reinterpret_cast<float (*)[kWave]>(&buf[0][0]);
+    importance_unit(job, (e - E) * (kWaves / 4) + wave / 4, red + wave / 4 * 4);
+    return;
+  }
   for (int i = tid; i < kWaves * E; i += kPlanThreads) hist[i / E][i % E] = 0;
   if (tid == 0) {
     s_fill = 0;
@@ -317,7 +322,7 @@ size_t plan_workspace_bytes(int64_t T, int64_t K, int64_t E) {
 int plan(const int32_t* top_idx, const float* top_w, int64_t T, int64_t K, int64_t E, int64_t capacity,
          int32_t* counts, int32_t* kept_counts, int32_t* kept_offsets, int32_t* slot_token, float* slot_weight,
          int32_t* route_slot, int32_t* dropped_token, int32_t* dropped_expert, int32_t* totals, void* ws,
-         size_t ws_bytes, hipStream_t stream) {
+         size_t ws_bytes, hipStream_t stream, const BalanceJob& job) {
   QW_REQUIRE(E >= 1 && E <= 1024, "experts must be in [1, 1024], got %lld", (long long)E);
   QW_REQUIRE(K >= 1 && K <= E, "top_k must be between 1 and num_experts");
   QW_REQUIRE(T >= 0 && T * K <= INT32_MAX, "tokens*top_k exceeds int32");
@@ -334,9 +339,11 @@ int plan(const int32_t* top_idx, const float* top_w, int64_t T, int64_t K, int64
   Carver c(ws);
   uint64_t* spill = c.take<uint64_t>(static_cast<size_t>(R));
   const int e = static_cast<int>(E);
-  plan_kernel<<<e, kPlanThreads, 0, stream>>>(top_idx, top_w, R, e, static_cast<int>(K), cap, counts, kept_counts,
+  // with a balance job of several 64-token chunks: extra workgroups for its partial sums
+  const int extra = job.nb > 1 ? static_cast<int>(ceil_div(partial_units(job.nb, e), kPlanThreads / kWave / 4)) : 0;
+  plan_kernel<<<e + extra, kPlanThreads, 0, stream>>>(top_idx, top_w, R, e, static_cast<int>(K), cap, counts, kept_counts,
                                               kept_offsets, totals, slot_token, slot_weight, route_slot, dropped_token,
-                                              dropped_expert, spill);
+                                              dropped_expert, spill, job);
   QW_LAUNCH_CHECK("plan_kernel");
   return QW_OK;
 }

@@ -512,22 +512,24 @@ class TopKMoE(nn.Module):
                 res = _layer_chain(flat, cdt, self.router.weight, self, pack, cap, bias, loop=loop, static=static)
         return self._finish(res["out"], res["probs"], res["balance"], res["top_idx"], res["top_w"], res["counts"],
                             res["kept_counts"], res["totals"], res["dropped_token"], res["dropped_expert"],
-                            token_domains, num_domains, (batch, sequence, width))
+                            token_domains, num_domains, (batch, sequence, width), res.get("overflow"),
+                            res.get("zero"))
 
     def _finish(self, out, probs, balance, top_idx, top_w, counts, kept_counts, totals, dropped_token, dropped_expert,
-                token_domains, num_domains, shape):
+                token_domains, num_domains, shape, overflow=None, zero=None):
+        """overflow, zero: the 64-bit dropped count and a zero, where the forward call wrote them."""
         dev = out.device
         self.last_top_indices = top_idx  # widened to int64 when read
         self.last_plan = dict(counts=counts, kept_counts=kept_counts, totals=totals, top_w=top_w,
                               dropped_token=dropped_token, dropped_expert=dropped_expert)
-        overflow_routes = totals[1].long()
+        overflow_routes = totals[1].long() if overflow is None else overflow
         if self.overflow_policy == "drop":
             dropped_routes = overflow_routes
         else:
             dropped_routes = torch.zeros((), device=dev, dtype=torch.long)
         if self.collect_stats and not self.static_dispatch:  # the dynamic path only (:141-149)
             self._record_stats(probs.detach(), top_idx, kept_counts, totals, dropped_token, dropped_expert)
-        domain_loss = probs.new_zeros(())
+        domain_loss = probs.new_zeros(()) if zero is None else zero
         if token_domains is not None and num_domains > 1:
             domain_loss = self._domain_loss(probs, token_domains, num_domains)
         return out.reshape(*shape), balance, dropped_routes, overflow_routes, domain_loss
@@ -579,39 +581,37 @@ def _forward_call(flat: Tensor, act: int, router_w: Tensor, moe: TopKMoE, pack: 
     R = T * K
     Rm = max(R, 1)
     rw = _router_operand(router_w)
-    # the per-call outputs in two slabs (int32 and fp32), handed out as views
-    ints = torch.empty(R + 2 * E + 2 + 2 * Rm, dtype=torch.int32, device=dev)
-    flts = torch.empty(T * E + R + 1 + E, dtype=torch.float32, device=dev)
-    top_idx, counts, kept_counts, totals, dropped_token, dropped_expert = ints.split([R, E, E, 2, Rm, Rm])
-    probs, top_w, balance, importance = flts.split([T * E, R, 1, E])
+    # the per-call outputs in two slabs (int32 and fp32), handed out as views;
+    # the first two int32 are the 64-bit overflow count
+    ints = torch.empty(2 + R + 2 * E + 2 + 2 * Rm, dtype=torch.int32, device=dev)
+    flts = torch.empty(T * E + R + 2 + E, dtype=torch.float32, device=dev)
+    overflow, top_idx, counts, kept_counts, totals, dropped_token, dropped_expert = ints.split([2, R, E, E, 2, Rm, Rm])
+    probs, top_w, balance, zero, importance = flts.split([T * E, R, 1, 1, E])
     r = dict(out=torch.empty_like(flat), probs=probs.view(T, E), top_w=top_w.view(T, K), balance=balance.view(()),
              top_idx=top_idx.view(T, K), counts=counts, kept_counts=kept_counts, totals=totals,
-             dropped_token=dropped_token, dropped_expert=dropped_expert)
+             dropped_token=dropped_token, dropped_expert=dropped_expert, overflow=overflow.view(torch.int64).view(()),
+             zero=zero.view(()))
     if not T:
-        totals.zero_()
-        balance.zero_()
+        ints[:2 + R + 2 * E + 2].zero_()
+        flts.zero_()
         return r
     key = (T, width, E, K, act)
     sizes = moe.__dict__.setdefault("_qw_sizes", {}).get(key)
     lib = _lib.load()
     if sizes is None:
         d_ff = moe.experts[0].gate.out_features
-        nbytes = lib.qw_moe_forward_workspace_bytes(T, width, E, K, d_ff, act)
-        fwd_bytes = (nbytes + 255) // 256 * 256
-        sizes = (d_ff, nbytes, fwd_bytes, lib.qw_moe_balance_workspace_bytes(T, E))
+        sizes = (d_ff, lib.qw_moe_forward_balance_workspace_bytes(T, width, E, K, d_ff, act))
         moe._qw_sizes[key] = sizes
-    d_ff, nbytes, fwd_bytes, bal_bytes = sizes
+    d_ff, nbytes = sizes
     s = torch.cuda.current_stream(dev).cuda_stream
-    ws = _stream_workspace(moe, fwd_bytes + bal_bytes, dev, s)
-    wp, ip, fp = ws.data_ptr(), ints.data_ptr(), flts.data_ptr()
-    p_probs, p_counts = fp, ip + 4 * (R + 0)
-    _lib.check(lib.qw_moe_forward(
+    wp = _stream_workspace(moe, nbytes, dev, s).data_ptr()
+    ip, fp = ints.data_ptr() + 8, flts.data_ptr()  # top_idx, probs
+    _lib.check(lib.qw_moe_forward_balance(
         flat.data_ptr(), act, T, width, rw.data_ptr(), _hip.act_code(rw, "router"), float(moe.router_temperature),
-        _hip.ptr(bias), E, K, cap, d_ff, *pack.args(), r["out"].data_ptr(), p_probs, ip, fp + 4 * T * E, p_counts,
-        ip + 4 * (R + E), ip + 4 * (R + 2 * E), ip + 4 * (R + 2 * E + 2), ip + 4 * (R + 2 * E + 2 + Rm), wp, nbytes,
-        s), "qw_moe_forward")
-    _lib.check(lib.qw_moe_balance_ws(p_probs, p_counts, T, K, E, fp + 4 * (T * E + R + 1), fp + 4 * (T * E + R), wp +
-                                     fwd_bytes, bal_bytes, s), "qw_moe_balance_ws")
+        _hip.ptr(bias), E, K, cap, d_ff, *pack.args(), r["out"].data_ptr(), fp, ip, fp + 4 * T * E, ip + 4 * R,
+        ip + 4 * (R + E), ip + 4 * (R + 2 * E), ip + 4 * (R + 2 * E + 2), ip + 4 * (R + 2 * E + 2 + Rm),
+        fp + 4 * (T * E + R + 2), fp + 4 * (T * E + R), ip - 8, fp + 4 * (T * E + R + 1), wp, nbytes, s),
+        "qw_moe_forward_balance")
     return r
 
 
