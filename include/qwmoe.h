@@ -123,6 +123,11 @@ int qw_moe_plan(const int32_t* top_idx, const float* top_w, int64_t tokens, int6
 int qw_moe_permute(const void* x, int dtype, int64_t d_model, const int32_t* slot_token, const int32_t* totals,
                    int64_t max_rows, void* out, void* stream);
 
+/* The same with the rows rounded to out_dtype: `flat.to(dtype)[tokens]`, what a
+ * mixed-precision backward pass gathers. */
+int qw_moe_permute_cast(const void* x, int dtype, int64_t d_model, const int32_t* slot_token, const int32_t* totals,
+                        int64_t max_rows, void* out, int out_dtype, void* stream);
+
 /* Grouped SwiGLU experts over plan-ordered rows.  Replaces
  * moe_kernels.grouped_swiglu (src/moe_kernels.py:186-195), the per-expert loop
  * (src/quantweave_moe_model.py:203-211) and, for quantised experts,
@@ -312,6 +317,15 @@ int qw_dequantize(const void* qweight, const float* scales, int bits, int64_t ou
 int qw_pack_bf16_tiles(const void* w, int64_t experts, int64_t out_features, int64_t in_features, void* tiled,
                        void* stream);
 
+/* The experts' own matrices [out_features, in_features] (src_dtype; a host
+ * array of device pointers, read during the call) -> one stack [experts,
+ * out_features, in_features] in out_format (QW_F32, QW_BF16, QW_F16, or the
+ * tiles QW_BF16T, QW_F16T), rounded to nearest even: the reference's per-call
+ * `stack(...).to(dtype)` (src/moe_kernels.py:191-193) and qw_pack_bf16_tiles in
+ * one pass.  in_features a multiple of 8, 16-byte aligned matrices. */
+int qw_pack_experts(const void* const* weights, int src_dtype, int64_t experts, int64_t out_features,
+                    int64_t in_features, void* out, int out_format, void* stream);
+
 /* Grouped matmul forward, moe_kernels.grouped_matmul (src/moe_kernels.py:118-135,
  * :167-171): out[rows of e] = x[rows of e] @ w[e]^T with rows of e =
  * [offsets[e], offsets[e+1]); w [E, out_features, in_features] in w_format
@@ -372,6 +386,14 @@ int qw_grouped_matmul_backward(const void* grad_out, const void* x, const void* 
                                int64_t out_features, int64_t in_features, const int32_t* offsets, int64_t rows,
                                int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x, void* grad_w,
                                int grad_w_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The same with the weights in w_format: `dtype`, or its tiles (QW_BF16T,
+ * QW_F16T), which the matrix-core grad_x reads as they are. */
+int qw_grouped_matmul_backward_fmt(const void* grad_out, const void* x, const void* w, int dtype, int w_format,
+                                   int64_t experts, int64_t out_features, int64_t in_features, const int32_t* offsets,
+                                   int64_t rows, int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x,
+                                   void* grad_w, int grad_w_dtype, void* workspace, size_t workspace_bytes,
+                                   void* stream);
 
 /* qw_moe_experts that also keeps what its backward needs, for training
  * (the activations autograd saves for SparseSwiGLU.forward,

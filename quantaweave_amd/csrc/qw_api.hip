@@ -46,6 +46,8 @@ int plan(const int32_t* top_idx, const float* top_w, int64_t T, int64_t K, int64
          size_t ws_bytes, hipStream_t stream, const BalanceJob& job = BalanceJob());
 int permute(const void* x, int dtype, int64_t D, const int32_t* slot_token, const int32_t* totals, int64_t max_rows,
             void* out, hipStream_t stream);
+int permute_cast(const void* x, int dtype, int64_t D, const int32_t* slot_token, const int32_t* totals,
+                 int64_t max_rows, void* out, int out_dtype, hipStream_t stream);
 int combine(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, int64_t T, int64_t K,
             int64_t D, void* out, hipStream_t stream);
 int decode_combine(const void* y, int dtype, const int32_t* route_slot, const float* top_w, const float* residual,
@@ -70,9 +72,11 @@ int combine_balance(const void* y, int dtype, const int32_t* route_slot, const i
                     hipStream_t stream);
 int combine_static(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
                    int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream);
-int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
-                            const int32_t* offsets, int64_t rows, int64_t max_rows_per_expert, void* gx, int accumulate,
-                            void* gw, int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream);
+int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int wfmt, int64_t E, int64_t N,
+                            int64_t K, const int32_t* offsets, int64_t rows, int64_t max_rows_per_expert, void* gx,
+                            int accumulate, void* gw, int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream);
+int pack_experts(const void* const* weights, int src, int64_t E, int64_t rows, int64_t cols, void* out, int fmt,
+                 hipStream_t stream);
 size_t grouped_backward_workspace_bytes(int64_t E, int64_t N, int64_t K, int64_t rows, int dtype);
 bool gemm_rows_fits(int64_t K, int64_t rows, int64_t E);
 int gemm_grouped_forward(const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
@@ -409,6 +413,12 @@ int qw_moe_permute(const void* x, int dtype, int64_t d_model, const int32_t* slo
                    int64_t max_rows, void* out, void* stream) {
   clear_error();
   return permute(x, dtype, d_model, slot_token, totals, max_rows, out, as_stream(stream));
+}
+
+int qw_moe_permute_cast(const void* x, int dtype, int64_t d_model, const int32_t* slot_token, const int32_t* totals,
+                        int64_t max_rows, void* out, int out_dtype, void* stream) {
+  clear_error();
+  return permute_cast(x, dtype, d_model, slot_token, totals, max_rows, out, out_dtype, as_stream(stream));
 }
 
 size_t qw_moe_experts_workspace_bytes(int64_t max_rows, int64_t experts, int64_t d_model, int64_t d_ff,
@@ -766,9 +776,26 @@ int qw_grouped_matmul_backward(const void* grad_out, const void* x, const void* 
                                int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x, void* grad_w,
                                int grad_w_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
-  return grouped_matmul_backward(grad_out, x, w, dtype, experts, out_features, in_features, offsets, rows,
+  return grouped_matmul_backward(grad_out, x, w, dtype, dtype, experts, out_features, in_features, offsets, rows,
                                  max_rows_per_expert, grad_x, accumulate_grad_x, grad_w, grad_w_dtype, workspace,
                                  workspace_bytes, as_stream(stream));
+}
+
+int qw_grouped_matmul_backward_fmt(const void* grad_out, const void* x, const void* w, int dtype, int w_format,
+                                   int64_t experts, int64_t out_features, int64_t in_features, const int32_t* offsets,
+                                   int64_t rows, int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x,
+                                   void* grad_w, int grad_w_dtype, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+  clear_error();
+  return grouped_matmul_backward(grad_out, x, w, dtype, w_format, experts, out_features, in_features, offsets, rows,
+                                 max_rows_per_expert, grad_x, accumulate_grad_x, grad_w, grad_w_dtype, workspace,
+                                 workspace_bytes, as_stream(stream));
+}
+
+int qw_pack_experts(const void* const* weights, int src_dtype, int64_t experts, int64_t out_features,
+                    int64_t in_features, void* out, int out_format, void* stream) {
+  clear_error();
+  return pack_experts(weights, src_dtype, experts, out_features, in_features, out, out_format, as_stream(stream));
 }
 
 int qw_swiglu(const void* gate, const void* up, int dtype, int64_t n, void* hidden, void* stream) {

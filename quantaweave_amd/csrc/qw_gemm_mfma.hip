@@ -20,6 +20,8 @@
 // tiles, fp32 accumulation, bf16 results.  Rows past the end of a group load
 // a valid row and are not stored.  The reduction in MODE_RED runs over
 // zero-padded slices (multiples of 64); an expert without rows gets zeros.
+#include <type_traits>
+
 #include "qw_common.h"
 
 namespace qw {
@@ -43,7 +45,7 @@ constexpr int G_XCDS = 8;                    // XCDs of the MI355X, workgroups d
 // quarter-wave reads at one logical piece land on 16 different bank groups.
 __device__ __forceinline__ int gswz(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-template <int DT, int MODE, bool ACCUM, bool BRED, bool C32>
+template <int DT, int MODE, bool ACCUM, bool BRED, bool C32, bool BT>
 __global__ __launch_bounds__(256) void gemm_nt_kernel(const uint16_t* __restrict__ A, int64_t lda,
                                                       const uint16_t* __restrict__ B, int64_t ldb,
                                                       int64_t b_expert_stride, void* __restrict__ C, int64_t ldc,
@@ -109,7 +111,16 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const uint16_t* __restrict
   // piece (8 reduction values) per column.  Columns past N read column N - 4
   // (in bounds, never stored).
   const int kg = tid % 32, ng = tid / 32;
-  const uint16_t* bt_src = b_base + static_cast<int64_t>(8 * ng) * ldb + min(n0 + 4 * kg, N - 4);
+  // BT: B in the 1 KiB tiles of QW_BF16T / QW_F16T: the eight rows are one tile's,
+  // row i at 64 i + 8 (piece ^ ((row / 2) % 8)); a slice of 64 rows advances as in
+  // the plain layout.
+  const int tc = min(n0 + 4 * kg, N - 4);
+  const uint16_t* bt_src = BT ? b_base + (static_cast<int64_t>(ng) * (N / 64) + tc / 64) * 512 + (tc & 7)
+                              : b_base + static_cast<int64_t>(8 * ng) * ldb + tc;
+  const int tpiece = (tc >> 3) & 7, tpar = 4 * (ng & 1);
+  auto bt_row = [&](int i) -> int64_t {
+    return BT ? 64 * i + 8 * (tpiece ^ (tpar + (i >> 1))) : static_cast<int64_t>(i) * ldb;
+  };
   uint4 ra0, ra1, ra2, ra3, rb0, rb1, rb2, rb3;
   uint2 rt0, rt1, rt2, rt3, rt4, rt5, rt6, rt7;
 #define QW_G_LOAD(kt)                                                        \
@@ -121,14 +132,14 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(const uint16_t* __restrict
     ra3 = *reinterpret_cast<const uint4*>(a_src[3] + k0_);                   \
     if (BRED) {                                                              \
       const uint16_t* t_ = bt_src + static_cast<int64_t>(k0_) * ldb;         \
-      rt0 = *reinterpret_cast<const uint2*>(t_);                             \
-      rt1 = *reinterpret_cast<const uint2*>(t_ + ldb);                       \
-      rt2 = *reinterpret_cast<const uint2*>(t_ + 2 * ldb);                   \
-      rt3 = *reinterpret_cast<const uint2*>(t_ + 3 * ldb);                   \
-      rt4 = *reinterpret_cast<const uint2*>(t_ + 4 * ldb);                   \
-      rt5 = *reinterpret_cast<const uint2*>(t_ + 5 * ldb);                   \
-      rt6 = *reinterpret_cast<const uint2*>(t_ + 6 * ldb);                   \
-      rt7 = *reinterpret_cast<const uint2*>(t_ + 7 * ldb);                   \
+      rt0 = *reinterpret_cast<const uint2*>(t_ + bt_row(0));                 \
+      rt1 = *reinterpret_cast<const uint2*>(t_ + bt_row(1));                 \
+      rt2 = *reinterpret_cast<const uint2*>(t_ + bt_row(2));                 \
+      rt3 = *reinterpret_cast<const uint2*>(t_ + bt_row(3));                 \
+      rt4 = *reinterpret_cast<const uint2*>(t_ + bt_row(4));                 \
+      rt5 = *reinterpret_cast<const uint2*>(t_ + bt_row(5));                 \
+      rt6 = *reinterpret_cast<const uint2*>(t_ + bt_row(6));                 \
+      rt7 = *reinterpret_cast<const uint2*>(t_ + bt_row(7));                 \
     } else {                                                                 \
       rb0 = *reinterpret_cast<const uint4*>(b_src[0] + k0_);                 \
       rb1 = *reinterpret_cast<const uint4*>(b_src[1] + k0_);                 \
@@ -444,11 +455,11 @@ __global__ __launch_bounds__(256) void transpose_pad_vec_kernel(const uint16_t* 
   }
 }
 
-template <int DT, int MODE, bool ACCUM, bool BRED = false, bool C32 = false>
+template <int DT, int MODE, bool ACCUM, bool BRED = false, bool C32 = false, bool BT = false>
 int launch_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t b_stride, void* C, int64_t ldc,
                 int64_t c_stride, const int32_t* offsets, int rows, int M, int N, int K, int E, int64_t m_extent,
                 hipStream_t stream) {
-  const hipError_t attr = reserve_lds<gemm_nt_kernel<DT, MODE, ACCUM, BRED, C32>>(G_LDS);
+  const hipError_t attr = reserve_lds<gemm_nt_kernel<DT, MODE, ACCUM, BRED, C32, BT>>(G_LDS);
   if (attr != hipSuccess) return set_error(QW_ERR_HIP, "cannot reserve LDS: %s", hipGetErrorString(attr));
   // one grid dimension: MODE_ROWS, the row tiles of all experts (at most
   // rows/128 + E) times the column tiles; MODE_RED, experts times output tiles;
@@ -457,7 +468,7 @@ int launch_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t 
   const int64_t blocks = MODE == MODE_ROWS ? G_XCDS * n_nt * ceil_div(ceil_div(m_extent, GT) + E, G_XCDS)
                                            : G_XCDS * n_nt * ceil_div(m_extent, GT) * ceil_div(E, G_XCDS);
   if (blocks > INT32_MAX) return set_error(QW_ERR_UNSUPPORTED, "grouped GEMM grid too large");
-  gemm_nt_kernel<DT, MODE, ACCUM, BRED, C32><<<static_cast<unsigned>(blocks), 256, G_LDS, stream>>>(
+  gemm_nt_kernel<DT, MODE, ACCUM, BRED, C32, BT><<<static_cast<unsigned>(blocks), 256, G_LDS, stream>>>(
       static_cast<const uint16_t*>(A), lda, static_cast<const uint16_t*>(B), ldb, b_stride, C, ldc, c_stride, offsets,
       rows, M, N, K, E);
   QW_LAUNCH_CHECK("gemm_nt_kernel");
@@ -502,8 +513,8 @@ int gemm_grouped_forward(const void* x, const void* w, int dtype, int64_t E, int
 //   gx = gy . w[e] (+ gx when accumulate), gw[e] = gy_e^T . x_e (fp32 when gw_f32).
 template <int DT>
 int gemm_backward_t(const void* gy, const void* x, const void* w, int64_t E, int64_t N, int64_t K,
-                    const int32_t* offsets, int64_t rows, void* gx, int accumulate, void* gw, int gw_f32, void* ws,
-                    size_t ws_bytes, hipStream_t stream) {
+                    const int32_t* offsets, int64_t rows, void* gx, int accumulate, void* gw, int gw_f32, bool tiled,
+                    void* ws, size_t ws_bytes, hipStream_t stream) {
   const size_t need = gemm_backward_workspace_bytes(E, N, K, rows);
   if (!ws || ws_bytes < need)
     return set_error(QW_ERR_WORKSPACE, "grouped backward workspace needs %zu bytes, got %zu", need, ws_bytes);
@@ -514,11 +525,13 @@ int gemm_backward_t(const void* gy, const void* x, const void* w, int64_t E, int
   int32_t* poff = c.take<int32_t>(E + 1);
   const int e = static_cast<int>(E), n = static_cast<int>(N), k = static_cast<int>(K), r = static_cast<int>(rows);
   if (gx != nullptr && rows > 0) {  // B = w read reduction-major: no transposed copy
-    const int st = accumulate
-                       ? launch_gemm<DT, MODE_ROWS, true, true>(gy, N, w, K, N * K, gx, K, 0, offsets, r, 0, k, n, e,
-                                                                rows, stream)
-                       : launch_gemm<DT, MODE_ROWS, false, true>(gy, N, w, K, N * K, gx, K, 0, offsets, r, 0, k, n, e,
-                                                                 rows, stream);
+    auto dx = [&](auto acc, auto bt) {
+      return launch_gemm<DT, MODE_ROWS, decltype(acc)::value, true, false, decltype(bt)::value>(
+          gy, N, w, K, N * K, gx, K, 0, offsets, r, 0, k, n, e, rows, stream);
+    };
+    using Y = std::true_type;
+    using No = std::false_type;
+    const int st = tiled ? (accumulate ? dx(Y{}, Y{}) : dx(No{}, Y{})) : (accumulate ? dx(Y{}, No{}) : dx(No{}, No{}));
     if (st) return st;
   }
   if (gw != nullptr) {
@@ -551,12 +564,13 @@ int gemm_backward_t(const void* gy, const void* x, const void* w, int64_t E, int
 
 int gemm_grouped_backward(const void* gy, const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
                           const int32_t* offsets, int64_t rows, int64_t rows_per_expert, void* gx, int accumulate,
-                          void* gw, int gw_f32, void* ws, size_t ws_bytes, hipStream_t stream) {
+                          void* gw, int gw_f32, bool tiled, void* ws, size_t ws_bytes, hipStream_t stream) {
   (void)rows_per_expert;
   if (dtype == QW_F16)
-    return gemm_backward_t<QW_F16>(gy, x, w, E, N, K, offsets, rows, gx, accumulate, gw, gw_f32, ws, ws_bytes,
-                                   stream);
-  return gemm_backward_t<QW_BF16>(gy, x, w, E, N, K, offsets, rows, gx, accumulate, gw, gw_f32, ws, ws_bytes, stream);
+    return gemm_backward_t<QW_F16>(gy, x, w, E, N, K, offsets, rows, gx, accumulate, gw, gw_f32, tiled, ws,
+                                   ws_bytes, stream);
+  return gemm_backward_t<QW_BF16>(gy, x, w, E, N, K, offsets, rows, gx, accumulate, gw, gw_f32, tiled, ws, ws_bytes,
+                                  stream);
 }
 
 }  // namespace qw

@@ -318,7 +318,7 @@ size_t gemm_backward_workspace_bytes(int64_t E, int64_t N, int64_t K, int64_t ro
 bool gemm_backward_fits(int64_t rows, int64_t E);
 int gemm_grouped_backward(const void* gy, const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
                           const int32_t* offsets, int64_t rows, int64_t rows_per_expert, void* gx, int accumulate,
-                          void* gw, int gw_f32, void* ws, size_t ws_bytes, hipStream_t stream);
+                          void* gw, int gw_f32, bool tiled, void* ws, size_t ws_bytes, hipStream_t stream);
 
 size_t grouped_backward_workspace_bytes(int64_t E, int64_t N, int64_t K, int64_t rows, int dtype) {
   return is_half(dtype) ? gemm_backward_workspace_bytes(E, N, K, rows) : 256;
@@ -326,14 +326,18 @@ size_t grouped_backward_workspace_bytes(int64_t E, int64_t N, int64_t K, int64_t
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int64_t E, int64_t N, int64_t K,
-                            const int32_t* offsets, int64_t rows, int64_t max_rows_per_expert, void* gx, int accumulate,
-                            void* gw, int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream) {
+int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int wfmt, int64_t E, int64_t N,
+                            int64_t K, const int32_t* offsets, int64_t rows, int64_t max_rows_per_expert, void* gx,
+                            int accumulate, void* gw, int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream) {
+  const bool tiled = wfmt != dtype;
   QW_REQUIRE(dtype == QW_F32 || dtype == QW_BF16 || dtype == QW_F16, "grouped backward dtype must be f32, bf16 or f16");
   QW_REQUIRE(gw_dtype == dtype || gw_dtype == QW_F32, "grad_w dtype must be the operands' dtype or f32");
   QW_REQUIRE(E >= 1 && E <= 65535 && N >= 1 && K >= 1 && N <= INT32_MAX && K <= INT32_MAX && rows >= 0 &&
                  rows <= INT32_MAX && max_rows_per_expert >= 0,
              "bad grouped backward sizes");
+  QW_REQUIRE(!tiled || (dtype == QW_BF16 && wfmt == QW_BF16T) || (dtype == QW_F16 && wfmt == QW_F16T),
+             "grouped backward weights must be of the operands' dtype, plain or tiled");
+  QW_REQUIRE(!tiled || (N % 64 == 0 && K % 64 == 0), "tiled weights need sizes that are multiples of 64");
   QW_REQUIRE(offsets != nullptr, "offsets are required");
   if (gx != nullptr && rows > 0) QW_REQUIRE(gy && w, "grad_x needs grad_out and w");
   if (gw != nullptr) QW_REQUIRE(rows == 0 || (gy && x), "grad_w needs grad_out and x");
@@ -346,11 +350,13 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   const bool core_dw = core && gw != nullptr && aligned16(gw);
   if (core_dx || core_dw) {
     const int st = gemm_grouped_backward(gy, x, w, dtype, E, N, K, offsets, rows, per, core_dx ? gx : nullptr, accumulate,
-                                         core_dw ? gw : nullptr, gw_dtype == QW_F32, ws, ws_bytes, stream);
+                                         core_dw ? gw : nullptr, gw_dtype == QW_F32, tiled, ws, ws_bytes, stream);
     if (st) return st;
     if (core_dx) gx = nullptr;
     if (core_dw) gw = nullptr;
   }
+  if (tiled && gx != nullptr && rows > 0)
+    return set_error(QW_ERR_UNSUPPORTED, "tiled weights need the matrix-core backward (workspace, aligned buffers)");
   const int n = static_cast<int>(N), k = static_cast<int>(K), r = static_cast<int>(rows);
   // fp32 matrix-core path: 16-byte rows and bases
   const bool f32_core = dtype == QW_F32 && N % 4 == 0 && K % 4 == 0 && aligned16(gy) && aligned16(x) &&

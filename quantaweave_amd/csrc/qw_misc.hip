@@ -41,6 +41,50 @@ int permute(const void* x, int dtype, int64_t D, const int32_t* slot_token, cons
   return QW_OK;
 }
 
+// The same with the rows rounded to another activation type on the way, eight
+// elements per thread and step (the cast of the whole input and its extra pass
+// over memory fall away: 20 us of 8192 x 2048 fp32 rows).
+template <int IN, int OUT, int VEC>
+__global__ __launch_bounds__(256) void permute_cast_kernel(const void* __restrict__ x, int D,
+                                                           const int32_t* __restrict__ slot_token,
+                                                           const int32_t* __restrict__ totals, int max_rows,
+                                                           void* __restrict__ out) {
+  const int s = blockIdx.x;
+  if (s >= min(*totals, max_rows)) return;
+  const int64_t src = static_cast<int64_t>(slot_token[s]) * D, dst = static_cast<int64_t>(s) * D;
+  for (int c = threadIdx.x * VEC; c < D; c += 256 * VEC) {
+    float v[VEC];
+    load_vec<IN, VEC>(x, src + c, v);
+    store_vec<OUT, VEC>(out, dst + c, v);
+  }
+}
+
+int permute_cast(const void* x, int dtype, int64_t D, const int32_t* slot_token, const int32_t* totals,
+                 int64_t max_rows, void* out, int out_dtype, hipStream_t stream) {
+  if (dtype == out_dtype) return permute(x, dtype, D, slot_token, totals, max_rows, out, stream);
+  QW_REQUIRE(D >= 1 && D <= INT32_MAX / 2 && max_rows >= 0 && max_rows <= INT32_MAX, "bad permute sizes");
+  if (max_rows == 0) return QW_OK;
+  QW_REQUIRE(x && slot_token && totals && out, "permute pointers are required");
+  const bool vec = D % 8 == 0 && (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0;
+  const unsigned g = static_cast<unsigned>(max_rows);
+  const int d = static_cast<int>(D), m = static_cast<int>(max_rows);
+#define QW_PC(I, O)                                                                                       \
+  if (dtype == I && out_dtype == O) {                                                                     \
+    if (vec) permute_cast_kernel<I, O, 8><<<g, 256, 0, stream>>>(x, d, slot_token, totals, m, out);       \
+    else permute_cast_kernel<I, O, 1><<<g, 256, 0, stream>>>(x, d, slot_token, totals, m, out);           \
+    QW_LAUNCH_CHECK("permute_cast_kernel");                                                               \
+    return QW_OK;                                                                                         \
+  }
+  QW_PC(QW_F32, QW_BF16)
+  QW_PC(QW_F32, QW_F16)
+  QW_PC(QW_BF16, QW_F32)
+  QW_PC(QW_BF16, QW_F16)
+  QW_PC(QW_F16, QW_F32)
+  QW_PC(QW_F16, QW_BF16)
+#undef QW_PC
+  return set_error(QW_ERR_INVALID, "permute dtypes must be f32, bf16 or f16 (got %d, %d)", dtype, out_dtype);
+}
+
 // ---------------------------------------------------------------------------
 // Combine: out[t] = the kept routes of t added in ascending expert order (the
 // plan order of `tokens`) in fp32, starting from zero, and rounded to the
@@ -448,6 +492,98 @@ int pack_bf16_tiles(const void* w, int64_t E, int64_t rows, int64_t cols, void* 
   pack_bf16_tiles_kernel<<<static_cast<unsigned>(ceil_div(pieces, 256)), 256, 0, stream>>>(
       static_cast<const uint16_t*>(w), pieces, rows, cols, static_cast<uint16_t*>(out));
   QW_LAUNCH_CHECK("pack_bf16_tiles_kernel");
+  return QW_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Experts' own weight matrices -> one stack [E, rows, cols], cast and tiled on
+// the way: what a training step needs after every weight update.  As torch
+// operations it was a stack, a cast and a packing pass per projection, and
+// another stack and cast for the backward (16 experts of 2048 x 1024 fp32:
+// 640 us a step); here each weight is read once and written once, at 16 bytes
+// per access, bound by HBM.  The matrices come as a table in the kernel's
+// arguments, so nothing is copied to the device first.
+// ---------------------------------------------------------------------------
+constexpr int kPackTable = 64;  // matrices per launch
+constexpr int kPackPieces = 4;  // 8-element pieces per thread
+
+struct PackTable {
+  const void* w[kPackTable];
+};
+
+template <int SRC, int DST, bool TILED>
+__global__ __launch_bounds__(256) void pack_experts_kernel(const PackTable table, int64_t pieces, int64_t cols,
+                                                           void* __restrict__ out) {
+  const void* const w = table.w[blockIdx.y];
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * (256 * kPackPieces) + threadIdx.x;
+  const int64_t base = static_cast<int64_t>(blockIdx.y) * pieces;  // the expert's first piece of the stack
+  float v[kPackPieces][8];
+#pragma unroll
+  for (int u = 0; u < kPackPieces; ++u) {
+    const int64_t o = first + 256 * u;
+    if (o >= pieces) break;
+    int64_t src = 8 * o;
+    if constexpr (TILED) {  // output piece o of the QW_BF16T tiles
+      const int64_t tile = o / 64, i = o % 64, kt = cols / 64;
+      const int64_t row = 8 * (tile / kt) + i / 8;
+      src = row * cols + (tile % kt) * 64 + ((i % 8) ^ ((row >> 1) & 7)) * 8;
+    }
+    load_vec<SRC, 8>(w, src, v[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kPackPieces; ++u) {
+    const int64_t o = first + 256 * u;
+    if (o >= pieces) break;
+    store_vec<DST, 8>(out, 8 * (base + o), v[u]);
+  }
+}
+
+int pack_experts(const void* const* weights, int src, int64_t E, int64_t rows, int64_t cols, void* out, int fmt,
+                 hipStream_t stream) {
+  QW_REQUIRE(E >= 1 && rows >= 1 && cols >= 1 && rows <= INT32_MAX / 2 && cols <= INT32_MAX / 2, "bad packing sizes");
+  QW_REQUIRE(weights && out, "packing pointers are required");
+  QW_REQUIRE(src == QW_F32 || src == QW_BF16 || src == QW_F16, "packed weights must be f32, bf16 or f16");
+  const bool tiled = fmt == QW_BF16T || fmt == QW_F16T;
+  const int dst = fmt == QW_BF16T ? QW_BF16 : fmt == QW_F16T ? QW_F16 : fmt;
+  QW_REQUIRE(dst == QW_F32 || dst == QW_BF16 || dst == QW_F16, "packing makes plain or tiled float stacks");
+  QW_REQUIRE(cols % 8 == 0 && (!tiled || (rows % 8 == 0 && cols % 64 == 0)),
+             "packing needs in_features %% 8 == 0, tiles out_features %% 8 == 0 and in_features %% 64 == 0");
+  QW_REQUIRE(reinterpret_cast<uintptr_t>(out) % 16 == 0, "packing needs 16-byte aligned buffers");
+  const int64_t pieces = rows * cols / 8;
+  const int64_t blocks = ceil_div(pieces, 256 * kPackPieces);
+  QW_REQUIRE(blocks <= INT32_MAX, "matrix too large to pack");
+  for (int64_t e0 = 0; e0 < E; e0 += kPackTable) {
+    PackTable t{};
+    const int n = static_cast<int>(E - e0 < kPackTable ? E - e0 : kPackTable);
+    for (int i = 0; i < n; ++i) {
+      t.w[i] = weights[e0 + i];
+      QW_REQUIRE(t.w[i] != nullptr && reinterpret_cast<uintptr_t>(t.w[i]) % 16 == 0,
+                 "packing needs 16-byte aligned matrices");
+    }
+    void* const to = static_cast<char*>(out) + e0 * rows * cols * (dst == QW_F32 ? 4 : 2);
+    const dim3 g(static_cast<unsigned>(blocks), static_cast<unsigned>(n));
+#define QW_PK(S, D, T)                                                            \
+  if (src == S && dst == D && tiled == T) {                                       \
+    pack_experts_kernel<S, D, T><<<g, 256, 0, stream>>>(t, pieces, cols, to);     \
+  }
+    QW_PK(QW_F32, QW_F32, false)
+    QW_PK(QW_F32, QW_BF16, false)
+    QW_PK(QW_F32, QW_BF16, true)
+    QW_PK(QW_F32, QW_F16, false)
+    QW_PK(QW_F32, QW_F16, true)
+    QW_PK(QW_BF16, QW_F32, false)
+    QW_PK(QW_BF16, QW_BF16, false)
+    QW_PK(QW_BF16, QW_BF16, true)
+    QW_PK(QW_BF16, QW_F16, false)
+    QW_PK(QW_BF16, QW_F16, true)
+    QW_PK(QW_F16, QW_F32, false)
+    QW_PK(QW_F16, QW_F16, false)
+    QW_PK(QW_F16, QW_F16, true)
+    QW_PK(QW_F16, QW_BF16, false)
+    QW_PK(QW_F16, QW_BF16, true)
+#undef QW_PK
+    QW_LAUNCH_CHECK("pack_experts_kernel");
+  }
   return QW_OK;
 }
 

@@ -101,11 +101,9 @@ def _expert_format(experts: nn.ModuleList) -> tuple[int, int, int]:
                     raise ValueError("all experts must share one quantisation format and group size")
         return fmt, g_in, g_ff
     dt = first.weight.dtype
-    for e in experts:
-        for name in ("gate", "up", "down"):
-            p = getattr(e, name)
-            if not isinstance(p, nn.Linear) or p.bias is not None or p.weight.dtype != dt:
-                raise ValueError("experts must be bias-free nn.Linear (one dtype) or QuantizedLinear projections")
+    for m in ExpertPack.projections(experts):
+        if not isinstance(m, nn.Linear) or m._parameters["bias"] is not None or m._parameters["weight"].dtype != dt:
+            raise ValueError("experts must be bias-free nn.Linear (one dtype) or QuantizedLinear projections")
     if dt not in _hip.FLOAT_DTYPES:
         raise ValueError(f"expert weight dtype {dt} is not supported (float32, bfloat16 or float16)")
     return _hip.act_code(first.weight, "experts"), 0, 0
@@ -126,6 +124,26 @@ def tile_bf16(stack: Tensor) -> Tensor:
 
 def can_tile(stack: Tensor) -> bool:
     return stack.dtype in _hip.HALF and stack.size(1) % 64 == 0 and stack.size(2) % 64 == 0
+
+
+def pack_weights(weights: list, dtype: torch.dtype, tile: bool) -> Tensor:
+    """The experts' own matrices [out, in] as one stack [E, out, in] of `dtype`,
+    in tiles if `tile` (16-bit, sizes of whole 64s): one kernel that reads each weight
+    once (qw_pack_experts); matrices it does not take (other devices, strides or
+    alignment) go through torch's stack and cast."""
+    w0 = weights[0]
+    rows, cols = w0.shape
+    ptrs = tuple(map(_DATA_PTR, weights))
+    native = w0.device.type == "cuda" and cols % 8 == 0 and w0.dtype in _hip.FLOAT_DTYPES and all(
+        w.dtype == w0.dtype and w.shape == w0.shape and w.device == w0.device and w.is_contiguous() for w in weights)
+    if not native or any(p % 16 for p in ptrs):
+        stack = torch.stack([w.detach() for w in weights]).to(dtype).contiguous()
+        return tile_bf16(stack) if tile else stack
+    out = torch.empty(len(weights), rows, cols, dtype=dtype, device=w0.device)
+    code = _hip.HALF[dtype][1] if tile else _hip.act_code(out, "pack_weights")
+    _lib.call("qw_pack_experts", (ctypes.c_void_p * len(ptrs))(*ptrs), _hip.act_code(w0, "pack_weights"), len(ptrs),
+              rows, cols, _hip.ptr(out), code, _hip.stream(w0.device))
+    return out
 
 
 # Every registration of a module, parameter or buffer anywhere in the process
@@ -185,11 +203,11 @@ class ExpertPack:
         self._quant = isinstance(self._exps[0]._modules["gate"], QuantizedLinear)
         self._token = None
         if self.fmt in (_lib.QW_F32, _lib.QW_BF16, _lib.QW_F16):
-            self.gate = torch.stack([e.gate.weight.detach() for e in experts]).contiguous()
-            self.up = torch.stack([e.up.weight.detach() for e in experts]).contiguous()
-            self.down = torch.stack([e.down.weight.detach() for e in experts]).contiguous()
             self.gate_s = self.up_s = self.down_s = None
-            self.maybe_tile()
+            self._float_weights = [[e._modules[n]._parameters["weight"].detach() for e in self._exps]
+                                   for n in ("gate", "up", "down")]
+            if self.fmt != _lib.QW_F32:  # fp32 stacks are made on first use: 16-bit arithmetic reads only its copies
+                self._stack_float()
         else:
             self.gate = torch.stack([e.gate.qweight for e in experts]).contiguous()
             self.up = torch.stack([e.up.qweight for e in experts]).contiguous()
@@ -204,6 +222,24 @@ class ExpertPack:
                         m = e._modules[name]
                         m.qweight, m.scales = q[i], sc[i]
         self._record(experts)
+
+    def _tileable(self) -> bool:
+        """The float experts' stacks can be tiles: all three projections, on a ROCm device."""
+        return all(w[0].device.type == "cuda" and w[0].size(0) % 64 == 0 and w[0].size(1) % 64 == 0
+                   for w in self._float_weights)
+
+    def _stack_float(self) -> None:
+        dt = self._float_weights[0][0].dtype
+        tile = dt in _hip.HALF and self._tileable()
+        self.gate, self.up, self.down = (pack_weights(w, dt, tile) for w in self._float_weights)
+        if tile:
+            self.fmt = _hip.HALF[dt][1]
+
+    def __getattr__(self, name: str):
+        if name in ("gate", "up", "down") and "_float_weights" in self.__dict__:
+            self._stack_float()
+            return self.__dict__[name]
+        raise AttributeError(name)
 
     def _record(self, experts: nn.ModuleList) -> None:
         """What ``current`` compares, as tuples built by C-level iteration (the
@@ -262,9 +298,14 @@ class ExpertPack:
             self.fmt = _lib.QW_BF16T if self.fmt == _lib.QW_BF16 else _lib.QW_F16T
 
     @staticmethod
+    def projections(experts: nn.ModuleList) -> list:
+        """gate, up and down of every expert, in order."""
+        return list(chain.from_iterable(map(_GATE_UP_DOWN, map(_SUBMODULES, experts._modules.values()))))
+
+    @staticmethod
     def sources(experts: nn.ModuleList) -> tuple[list, list]:
         """The projection modules and the tensors the pack was made from."""
-        mods = [m for e in experts._modules.values() for m in (e._modules["gate"], e._modules["up"], e._modules["down"])]
+        mods = ExpertPack.projections(experts)
         tensors = []
         for m in mods:
             if isinstance(m, QuantizedLinear):
@@ -301,16 +342,23 @@ class ExpertPack:
             self._args = cached
         return cached[1]
 
-    def plain(self, experts: nn.ModuleList, dtype: torch.dtype) -> list:
-        """[gate, up, down] stacks [E, out, in] in `dtype`, untiled, for the
-        backward kernels; made once per weight version."""
-        cache = getattr(self, "_plain", None)
+    def backward_operands(self, dtype: torch.dtype, rows: int) -> tuple[int, list]:
+        """(format, [gate, up, down] stacks [E, out, in]) in `dtype` for the
+        backward kernels on `rows` rows: the stacks the forward multiplied,
+        tiles included."""
+        src = self.for_act(_hip.act_code(torch.empty(0, dtype=dtype), "backward"))
+        code = _hip.act_code(torch.empty(0, dtype=dtype), "backward")
+        stacks = [src.gate, src.up, src.down]
+        if src.fmt == code:
+            return code, stacks
+        # tiles of this type, as long as the matrix-core backward's grid holds the rows
+        if dtype in _hip.HALF and src.fmt == _hip.HALF[dtype][1] and -(-rows // 64) + stacks[0].size(0) <= 65535:
+            return src.fmt, stacks
+        cache = self.__dict__.get("_plain")
         if cache is None or cache[0] != dtype:
-            stacks = [torch.stack([getattr(e, n).weight.detach() for e in experts]).to(dtype).contiguous()
-                      for n in ("gate", "up", "down")]
-            cache = (dtype, stacks)
+            cache = (dtype, [pack_weights(w, dtype, False) for w in self._float_weights])
             self._plain = cache
-        return cache[1]
+        return code, cache[1]
 
     def args_for(self, act: int) -> list:
         """Weight arguments for activations of dtype code `act`: float experts
@@ -331,15 +379,21 @@ class ExpertPack:
         if act not in copies:
             dt = torch.bfloat16 if act == _lib.QW_BF16 else torch.float16
             cast = ExpertPack.__new__(ExpertPack)
-            cast.group_in, cast.group_ff = 0, 0
-            # tiles are a permutation of the elements: a cast keeps them tiles
-            cast.gate, cast.up, cast.down = (t.to(dt).contiguous() for t in (self.gate, self.up, self.down))
+            cast.fmt, cast.group_in, cast.group_ff = act, 0, 0
             cast.gate_s = cast.up_s = cast.down_s = None
-            if self.fmt in plain_of:
-                cast.fmt = _lib.QW_BF16T if act == _lib.QW_BF16 else _lib.QW_F16T
+            # the masters, or a decode step's stacks moved to its device
+            if "gate" in self.__dict__ and self.gate.device != self._float_weights[0][0].device:
+                # tiles are a permutation of the elements: a cast keeps them tiles
+                cast.gate, cast.up, cast.down = (t.to(dt).contiguous() for t in (self.gate, self.up, self.down))
+                if self.fmt in plain_of:
+                    cast.fmt = _hip.HALF[dt][1]
+                else:
+                    cast.maybe_tile()
             else:
-                cast.fmt = act
-                cast.maybe_tile()
+                tile = self._tileable()
+                cast.gate, cast.up, cast.down = (pack_weights(w, dt, tile) for w in self._float_weights)
+                if tile:
+                    cast.fmt = _hip.HALF[dt][1]
             copies[act] = cast
         return copies[act]
 
@@ -787,20 +841,21 @@ class _MoELayer(torch.autograd.Function):
             _lib.call("qw_moe_combine_backward", _hip.ptr(d_out), act_in, _hip.ptr(y), act, _hip.ptr(route_slot),
                       _hip.ptr(top_w), T, K, D, _hip.ptr(dy), _hip.ptr(d_top_w), s)
             if need_x or need_experts:
-                stacks = ctx.pack.plain(moe.experts, cdt)
+                wfmt, stacks = ctx.pack.backward_operands(cdt, R)
                 plan = _RowPlan(kept_offsets, E, min(ctx.cap, R))
                 xp = torch.empty(R, D, dtype=cdt, device=dev)
-                _lib.call("qw_moe_permute", _hip.ptr(flat.to(cdt)), act, D, _hip.ptr(slot_token), _hip.ptr(totals), R,
-                          _hip.ptr(xp), s)
+                _lib.call("qw_moe_permute_cast", _hip.ptr(flat), act_in, D, _hip.ptr(slot_token), _hip.ptr(totals), R,
+                          _hip.ptr(xp), act, s)
                 wdt = moe.experts[0].gate.weight.dtype  # fp32 parameters: unrounded fp32 gradients
                 gwd = torch.float32 if wdt == torch.float32 else None
-                dh, d_down = _backward(dy, h, stacks[2], plan, act, True, need_experts, grad_w_dtype=gwd)
+                dh, d_down = _backward(dy, h, stacks[2], plan, act, True, need_experts, grad_w_dtype=gwd, w_format=wfmt)
                 dg, du = torch.empty_like(g), torch.empty_like(u)
                 _lib.call("qw_swiglu_backward", _hip.ptr(dh), _hip.ptr(g), _hip.ptr(u), act, g.numel(), _hip.ptr(dg),
                           _hip.ptr(du), s)
-                dxp, d_gate = _backward(dg, xp, stacks[0], plan, act, need_x, need_experts, grad_w_dtype=gwd)
+                dxp, d_gate = _backward(dg, xp, stacks[0], plan, act, need_x, need_experts, grad_w_dtype=gwd,
+                                        w_format=wfmt)
                 dxp, d_up = _backward(du, xp, stacks[1], plan, act, need_x, need_experts, grad_x=dxp,
-                                      grad_w_dtype=gwd)
+                                      grad_w_dtype=gwd, w_format=wfmt)
                 if need_experts:
                     for j, (n, gw) in enumerate((("gate", d_gate), ("up", d_up), ("down", d_down))):
                         per = gw.to(getattr(moe.experts[0], n).weight.dtype).unbind(0)
@@ -821,8 +876,12 @@ class _MoELayer(torch.autograd.Function):
             if need_router:
                 d_router = (d_scores.t() @ flat.float()).to(ctx.router_dtype)
             if need_x:
-                dx_router = (d_scores @ rw.float()).to(flat.dtype)
-                d_flat = dx_router if d_flat is None else d_flat + dx_router
+                if d_flat is None:
+                    d_flat = (d_scores @ rw.float()).to(flat.dtype)
+                elif d_flat.dtype == torch.float32:
+                    d_flat.addmm_(d_scores, rw.float())  # one pass over d_flat: product and sum
+                else:
+                    d_flat = d_flat + (d_scores @ rw.float()).to(flat.dtype)
         return (d_flat, d_router, None, None, None, None, None, None, None, *expert_grads)
 
 

@@ -90,11 +90,12 @@ def _forward(x: Tensor, w: Tensor, plan: GroupedPlan, act: int) -> Tensor:
 
 
 def _backward(grad: Tensor, x: Tensor, w: Tensor, plan: GroupedPlan, act: int, need_x: bool, need_w: bool,
-              grad_x: Optional[Tensor] = None, grad_w_dtype: Optional[torch.dtype] = None
-              ) -> tuple[Optional[Tensor], Optional[Tensor]]:
+              grad_x: Optional[Tensor] = None, grad_w_dtype: Optional[torch.dtype] = None,
+              w_format: Optional[int] = None) -> tuple[Optional[Tensor], Optional[Tensor]]:
     """(grad_x, grad_w) of out = grouped x @ w^T.  A given grad_x is added to.
     grad_w_dtype: float32 to get the weight gradient unrounded (fp32
-    parameters multiplied in bf16); default the operands' dtype."""
+    parameters multiplied in bf16); default the operands' dtype.  w_format:
+    the tiles' format code when w holds them."""
     gx = gw = None
     accumulate = grad_x is not None
     if need_x:
@@ -105,7 +106,8 @@ def _backward(grad: Tensor, x: Tensor, w: Tensor, plan: GroupedPlan, act: int, n
     if gx is not None or gw is not None:
         nbytes = _lib.load().qw_grouped_matmul_backward_workspace_bytes(w.size(0), w.size(1), w.size(2), x.size(0), act)
         ws = _hip.workspace(nbytes, x.device)
-        _lib.call("qw_grouped_matmul_backward", _hip.ptr(grad), _hip.ptr(x), _hip.ptr(w), act, w.size(0), w.size(1),
+        _lib.call("qw_grouped_matmul_backward_fmt", _hip.ptr(grad), _hip.ptr(x), _hip.ptr(w), act,
+                  act if w_format is None else w_format, w.size(0), w.size(1),
                   w.size(2), _hip.ptr(plan.offsets), x.size(0), plan.max_count, _hip.ptr(gx), int(accumulate),
                   _hip.ptr(gw), _hip.act_code(torch.empty(0, dtype=gw_dtype), "grad_w"), _hip.ptr(ws), nbytes,
                   _hip.stream(x.device))
@@ -215,7 +217,7 @@ def grouped_swiglu(inputs: Tensor, experts: nn.ModuleList, counts: Sequence[int]
     # the reference casts the stacked weights to the compute dtype (src/moe_kernels.py:191-193);
     # bf16 weights under fp32 activations are widened exactly inside the kernels
     args = pack.args_for(act)
-    d_ff = pack.gate.size(1)
+    d_ff = experts[0].gate.out_features
     d_model = x.size(1)
     out = torch.empty(plan.rows, d_model, dtype=dtype, device=x.device)
     if plan.rows:
