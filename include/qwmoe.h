@@ -376,10 +376,12 @@ int qw_moe_combine_static(const void* y, int y_dtype, const int32_t* route_slot,
  * in bf16 (the gradient is then not rounded to bf16).
  * accumulate_grad_x != 0 adds to grad_x instead of overwriting it.
  * max_rows_per_expert bounds every expert's row count (0: `rows`).
- * bf16 or fp16 with a workspace of qw_grouped_matmul_backward_workspace_bytes runs on
- * the matrix cores (grad_x when out_features % 64 == 0; grad_w always): the
- * weights and the row blocks are transposed into the workspace first.  fp32,
- * or no workspace, runs the vector-ALU kernels. */
+ * bf16 or fp16 runs on the matrix cores, on the operands as they lie where the
+ * sizes are multiples of 8 and fill 256-column tiles (in_features >= 192; grad_x:
+ * out_features % 64 == 0, not accumulating; grad_w: out_features >= 96), else
+ * with a workspace of qw_grouped_matmul_backward_workspace_bytes (grad_x when
+ * out_features % 64 == 0; grad_w always: the row blocks are transposed into the
+ * workspace first), else on the vector-ALU kernels. */
 size_t qw_grouped_matmul_backward_workspace_bytes(int64_t experts, int64_t out_features, int64_t in_features,
                                                   int64_t rows, int dtype);
 int qw_grouped_matmul_backward(const void* grad_out, const void* x, const void* w, int dtype, int64_t experts,
@@ -394,6 +396,17 @@ int qw_grouped_matmul_backward_fmt(const void* grad_out, const void* x, const vo
                                    int64_t rows, int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x,
                                    void* grad_w, int grad_w_dtype, void* workspace, size_t workspace_bytes,
                                    void* stream);
+
+/* The backward of two products of the same x (the gate and up projections):
+ * grad_x[r] = grad_out_a[r] @ w_a[e] + grad_out_b[r] @ w_b[e], and both weight
+ * gradients.  grad_x, grad_w_a or grad_w_b may be NULL.  Other arguments as
+ * above; grad_x is overwritten, summed in fp32 and rounded once where the
+ * 256-column tiles apply, else as two calls, the second accumulating. */
+int qw_grouped_matmul_backward_pair(const void* grad_out_a, const void* grad_out_b, const void* x, const void* w_a,
+                                    const void* w_b, int dtype, int w_format, int64_t experts, int64_t out_features,
+                                    int64_t in_features, const int32_t* offsets, int64_t rows,
+                                    int64_t max_rows_per_expert, void* grad_x, void* grad_w_a, void* grad_w_b,
+                                    int grad_w_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* qw_moe_experts that also keeps what its backward needs, for training
  * (the activations autograd saves for SparseSwiGLU.forward,

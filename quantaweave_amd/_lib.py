@@ -62,6 +62,8 @@ SIGNATURES = {
     "qw_moe_permute_cast": (I32, [P, I32, I64, P, P, I64, P, I32, P]),
     "qw_pack_experts": (I32, [P, I32, I64, I64, I64, P, I32, P]),
     "qw_grouped_matmul_backward_fmt": (I32, [P, P, P, I32, I32, I64, I64, I64, P, I64, I64, P, I32, P, I32, P, SZ, P]),
+    "qw_grouped_matmul_backward_pair": (I32, [P, P, P, P, P, I32, I32, I64, I64, I64, P, I64, I64, P, P, P, I32, P, SZ,
+                                              P]),
     "qw_grouped_matmul_backward": (I32, [P, P, P, I32, I64, I64, I64, P, I64, I64, P, I32, P, I32, P, SZ, P]),
     "qw_moe_experts_save": (I32, [P, I32, P, P, I64, I64, I64, I64, I64, I32, I64, I64, P, P, P, P, P, P, P, P,
                                   P, P, P, P, P, SZ, P]),

@@ -72,6 +72,10 @@ int combine_balance(const void* y, int dtype, const int32_t* route_slot, const i
                     hipStream_t stream);
 int combine_static(const void* y, int dtype, const int32_t* route_slot, const int32_t* top_idx, const float* top_w,
                    int64_t T, int64_t K, int64_t D, void* out, int out_dtype, hipStream_t stream);
+int grouped_matmul_backward_pair(const void* gy_a, const void* gy_b, const void* x, const void* w_a, const void* w_b,
+                                 int dtype, int wfmt, int64_t E, int64_t N, int64_t K, const int32_t* offsets,
+                                 int64_t rows, int64_t max_rows_per_expert, void* gx, void* gw_a, void* gw_b,
+                                 int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream);
 int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dtype, int wfmt, int64_t E, int64_t N,
                             int64_t K, const int32_t* offsets, int64_t rows, int64_t max_rows_per_expert, void* gx,
                             int accumulate, void* gw, int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream);
@@ -790,6 +794,17 @@ int qw_grouped_matmul_backward_fmt(const void* grad_out, const void* x, const vo
   return grouped_matmul_backward(grad_out, x, w, dtype, w_format, experts, out_features, in_features, offsets, rows,
                                  max_rows_per_expert, grad_x, accumulate_grad_x, grad_w, grad_w_dtype, workspace,
                                  workspace_bytes, as_stream(stream));
+}
+
+int qw_grouped_matmul_backward_pair(const void* grad_out_a, const void* grad_out_b, const void* x, const void* w_a,
+                                    const void* w_b, int dtype, int w_format, int64_t experts, int64_t out_features,
+                                    int64_t in_features, const int32_t* offsets, int64_t rows,
+                                    int64_t max_rows_per_expert, void* grad_x, void* grad_w_a, void* grad_w_b,
+                                    int grad_w_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  return grouped_matmul_backward_pair(grad_out_a, grad_out_b, x, w_a, w_b, dtype, w_format, experts, out_features,
+                                      in_features, offsets, rows, max_rows_per_expert, grad_x, grad_w_a, grad_w_b,
+                                      grad_w_dtype, workspace, workspace_bytes, as_stream(stream));
 }
 
 int qw_pack_experts(const void* const* weights, int src_dtype, int64_t experts, int64_t out_features,

@@ -320,6 +320,13 @@ int gemm_grouped_backward(const void* gy, const void* x, const void* w, int dtyp
                           const int32_t* offsets, int64_t rows, int64_t rows_per_expert, void* gx, int accumulate,
                           void* gw, int gw_f32, bool tiled, void* ws, size_t ws_bytes, hipStream_t stream);
 
+bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows);
+int gemm_tr_dx(const void* gy0, const void* gy1, const void* w0, const void* w1, int dtype, bool tiled, int64_t E,
+               int64_t N, int64_t K, const int32_t* offsets, int64_t rows, void* gx, hipStream_t stream);
+bool gemm_tr_dw_fits(const void* gy, const void* x, const void* gw, int64_t E, int64_t N, int64_t K);
+int gemm_tr_dw(const void* gy0, const void* gy1, const void* x, int dtype, int64_t E, int64_t N, int64_t K,
+               const int32_t* offsets, int64_t rows, void* gw0, void* gw1, int gw_f32, hipStream_t stream);
+
 size_t grouped_backward_workspace_bytes(int64_t E, int64_t N, int64_t K, int64_t rows, int dtype) {
   return is_half(dtype) ? gemm_backward_workspace_bytes(E, N, K, rows) : 256;
 }
@@ -343,6 +350,17 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   if (gw != nullptr) QW_REQUIRE(rows == 0 || (gy && x), "grad_w needs grad_out and x");
   const int64_t per = max_rows_per_expert > 0 && max_rows_per_expert < rows ? max_rows_per_expert : rows;
   QW_REQUIRE(ceil_div(per, BT) <= 65535 && ceil_div(N, BT) <= 65535, "grouped backward sizes out of range");
+  // 256-column tiles over the operands as they lie (no workspace)
+  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && gemm_tr_dx_fits(gy, w, gx, E, N, K, rows)) {
+    const int st = gemm_tr_dx(gy, nullptr, w, nullptr, dtype, tiled, E, N, K, offsets, rows, gx, stream);
+    if (st) return st;
+    gx = nullptr;
+  }
+  if (is_half(dtype) && gw != nullptr && gemm_tr_dw_fits(gy, x, gw, E, N, K)) {
+    const int st = gemm_tr_dw(gy, nullptr, x, dtype, E, N, K, offsets, rows, gw, nullptr, gw_dtype == QW_F32, stream);
+    if (st) return st;
+    gw = nullptr;
+  }
   // matrix-core path (bf16/fp16 with a workspace): dX needs out_features % 64 == 0, dW any shape
   const bool core = is_half(dtype) && ws != nullptr && ws_bytes >= gemm_backward_workspace_bytes(E, N, K, rows) &&
                     aligned16(gy) && aligned16(x) && aligned16(w) && gemm_backward_fits(rows, E);
@@ -397,6 +415,39 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
     QW_LAUNCH_CHECK("grouped_dw_kernel");
   }
   return QW_OK;
+}
+
+// Two products of the same x: gx = gy_a . w_a + gy_b . w_b, gw_a and gw_b.
+int grouped_matmul_backward_pair(const void* gy_a, const void* gy_b, const void* x, const void* w_a, const void* w_b,
+                                 int dtype, int wfmt, int64_t E, int64_t N, int64_t K, const int32_t* offsets,
+                                 int64_t rows, int64_t max_rows_per_expert, void* gx, void* gw_a, void* gw_b,
+                                 int gw_dtype, void* ws, size_t ws_bytes, hipStream_t stream) {
+  // the checks of the single product, which launches nothing here
+  int st = grouped_matmul_backward(gy_a, x, w_a, dtype, wfmt, E, N, K, offsets, rows, max_rows_per_expert, nullptr, 0,
+                                   nullptr, gw_dtype, ws, ws_bytes, stream);
+  if (st) return st;
+  if (gx != nullptr && rows > 0) QW_REQUIRE(gy_a && gy_b && w_a && w_b, "grad_x needs grad_out and w");
+  if (gw_a != nullptr || gw_b != nullptr) QW_REQUIRE(rows == 0 || (gy_a && gy_b && x), "grad_w needs grad_out and x");
+  // one accumulator for both: one rounding instead of two, and grad_x written once
+  if (is_half(dtype) && gx != nullptr && rows > 0 && gemm_tr_dx_fits(gy_a, w_a, gx, E, N, K, rows) &&
+      gemm_tr_dx_fits(gy_b, w_b, gx, E, N, K, rows)) {
+    st = gemm_tr_dx(gy_a, gy_b, w_a, w_b, dtype, wfmt != dtype, E, N, K, offsets, rows, gx, stream);
+    if (st) return st;
+    gx = nullptr;
+  }
+  if (is_half(dtype) && gw_a != nullptr && gw_b != nullptr && gemm_tr_dw_fits(gy_a, x, gw_a, E, N, K) &&
+      gemm_tr_dw_fits(gy_b, x, gw_b, E, N, K)) {
+    st = gemm_tr_dw(gy_a, gy_b, x, dtype, E, N, K, offsets, rows, gw_a, gw_b, gw_dtype == QW_F32, stream);
+    if (st) return st;
+    gw_a = gw_b = nullptr;
+  }
+  if (gx != nullptr || gw_a != nullptr)
+    st = grouped_matmul_backward(gy_a, x, w_a, dtype, wfmt, E, N, K, offsets, rows, max_rows_per_expert, gx, 0, gw_a,
+                                 gw_dtype, ws, ws_bytes, stream);
+  if (!st && (gx != nullptr || gw_b != nullptr))
+    st = grouped_matmul_backward(gy_b, x, w_b, dtype, wfmt, E, N, K, offsets, rows, max_rows_per_expert, gx, 1, gw_b,
+                                 gw_dtype, ws, ws_bytes, stream);
+  return st;
 }
 
 }  // namespace qw

@@ -834,7 +834,7 @@ class _MoELayer(torch.autograd.Function):
         expert_grads = [None] * n_w
         d_top_w = torch.zeros(T, K, dtype=torch.float32, device=dev)
         if T and d_out is not None and (need_x or need_router or need_experts):
-            from .moe_kernels import _backward
+            from .moe_kernels import _backward, _backward_pair
 
             d_out = d_out.contiguous().to(flat.dtype)
             dy = torch.empty_like(y)
@@ -852,10 +852,8 @@ class _MoELayer(torch.autograd.Function):
                 dg, du = torch.empty_like(g), torch.empty_like(u)
                 _lib.call("qw_swiglu_backward", _hip.ptr(dh), _hip.ptr(g), _hip.ptr(u), act, g.numel(), _hip.ptr(dg),
                           _hip.ptr(du), s)
-                dxp, d_gate = _backward(dg, xp, stacks[0], plan, act, need_x, need_experts, grad_w_dtype=gwd,
-                                        w_format=wfmt)
-                dxp, d_up = _backward(du, xp, stacks[1], plan, act, need_x, need_experts, grad_x=dxp,
-                                      grad_w_dtype=gwd, w_format=wfmt)
+                dxp, d_gate, d_up = _backward_pair((dg, du), xp, stacks[:2], plan, act, need_x,
+                                                   (need_experts, need_experts), grad_w_dtype=gwd, w_format=wfmt)
                 if need_experts:
                     for j, (n, gw) in enumerate((("gate", d_gate), ("up", d_up), ("down", d_down))):
                         per = gw.to(getattr(moe.experts[0], n).weight.dtype).unbind(0)

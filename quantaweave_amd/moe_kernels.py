@@ -114,6 +114,25 @@ def _backward(grad: Tensor, x: Tensor, w: Tensor, plan: GroupedPlan, act: int, n
     return gx, gw
 
 
+def _backward_pair(grads: Sequence[Tensor], x: Tensor, ws: Sequence[Tensor], plan: GroupedPlan, act: int, need_x: bool,
+                   need_w: Sequence[bool], grad_w_dtype: Optional[torch.dtype] = None,
+                   w_format: Optional[int] = None) -> tuple:
+    """(grad_x, grad_w of the first, of the second) of two products of the same x (see _backward)."""
+    w = ws[0]
+    gw_dtype = w.dtype if grad_w_dtype is None else grad_w_dtype
+    gx = torch.empty_like(x) if need_x else None
+    gws = [torch.empty(w.shape, dtype=gw_dtype, device=w.device) if need else None for need in need_w]
+    if need_x or any(need_w):
+        nbytes = _lib.load().qw_grouped_matmul_backward_workspace_bytes(w.size(0), w.size(1), w.size(2), x.size(0), act)
+        space = _hip.workspace(nbytes, x.device)
+        _lib.call("qw_grouped_matmul_backward_pair", _hip.ptr(grads[0]), _hip.ptr(grads[1]), _hip.ptr(x),
+                  _hip.ptr(ws[0]), _hip.ptr(ws[1]), act, act if w_format is None else w_format, w.size(0), w.size(1),
+                  w.size(2), _hip.ptr(plan.offsets), x.size(0), plan.max_count, _hip.ptr(gx), _hip.ptr(gws[0]),
+                  _hip.ptr(gws[1]), _hip.act_code(torch.empty(0, dtype=gw_dtype), "grad_w"), _hip.ptr(space), nbytes,
+                  _hip.stream(x.device))
+    return gx, *gws
+
+
 class _GroupedMatmul(torch.autograd.Function):
     """src/moe_kernels.py:138-164: grad_x = grad_out @ W[e] per expert block,
     grad_W[e] = grad_out[rows of e]^T @ x[rows of e] (exactly zero for an
@@ -149,8 +168,8 @@ class _GroupedSwiGLU(torch.autograd.Function):
     """down(silu(gate(x)) * up(x)) over expert blocks with its backward, the
     composition grouped_swiglu builds from _GroupedMatmul and F.silu
     (src/moe_kernels.py:186-195): three grouped matmuls and qw_swiglu forward;
-    qw_swiglu_backward and five grouped backward products (grad_x of gate and
-    up summed in place) backward.  Weights are stacked [E, out, in] of x's dtype."""
+    qw_swiglu_backward and the grouped backward products (grad_x of gate and
+    up as one sum) backward.  Weights are stacked [E, out, in] of x's dtype."""
 
     @staticmethod
     def forward(ctx, x: Tensor, gate: Tensor, up: Tensor, down: Tensor, plan: GroupedPlan) -> Tensor:
@@ -176,8 +195,7 @@ class _GroupedSwiGLU(torch.autograd.Function):
         dg, du = torch.empty_like(g), torch.empty_like(u)
         _lib.call("qw_swiglu_backward", _hip.ptr(dh), _hip.ptr(g), _hip.ptr(u), act, g.numel(), _hip.ptr(dg),
                   _hip.ptr(du), _hip.stream(x.device))
-        dx, d_gate = _backward(dg, x, gate, plan, act, need_x, need_g)
-        dx, d_up = _backward(du, x, up, plan, act, need_x, need_u, grad_x=dx)
+        dx, d_gate, d_up = _backward_pair((dg, du), x, (gate, up), plan, act, need_x, (need_g, need_u))
         return dx, d_gate, d_up, d_down, None
 
 
