@@ -38,7 +38,6 @@ constexpr int TR_THREADS = 512, TR_WAVES = 8;
 constexpr int TR_N = 256;   // columns per tile
 constexpr int TR_K = 64;    // reduction slice
 constexpr int TR_LDS = 160 * 1024;
-constexpr int TR_CUS = 256;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
@@ -293,18 +292,30 @@ int launch_tr(const TrArgs& a, int64_t blocks, hipStream_t stream) {
   return QW_OK;
 }
 
-// Rounds of one workgroup per compute unit, a 256-row tile counted as two 128-row ones.
-bool tall_tiles(double tiles256, double tiles128) {
-  auto rounds = [](double t) { return std::ceil(t / TR_CUS); };
-  return 2.0 * rounds(tiles256) <= 1.15 * rounds(tiles128);
-}
+// 256-row tiles where they come near filling the compute units once (`tiles`, one
+// workgroup each), else 128-row ones.  Measured on 2048 x 1024 to 256 x 512
+// matrices of 8 to 32 experts, 4000 and 16000 rows: 216 tiles dX 36.7 us against
+// 46.2 (128 rows), 282 tiles 48.6 against 70.9, 512 tiles dW 75 against 113;
+// 189 tiles dX 34.8 against 28.6, 64 tiles dW 56 against 39.
+bool tall_tiles(double tiles) { return tiles >= 200; }
+
+// Row tiles of all experts at `height` rows: on average half a tile per expert is a remainder.
+double row_tiles(int64_t rows, int64_t E, int height) { return static_cast<double>(rows) / height + 0.5 * E; }
 
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
 
 // dX of one product, or of two summed (gy1, w1 non-null): N columns of gy are the reduction.
-bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows) {
+bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows,
+                     bool pair) {
+  // One product: 128 x 128 tiles (gemm_nt_kernel) are level or faster where 256-row
+  // tiles do not fill the chip (1024 x 2048, 16 experts, 4000 rows: 28.0 us against
+  // 28.6; 512 x 256, 16000 rows: 14.4 against 15.7), except below 96 rows an
+  // expert, where whole sub-tiles are skipped (1000 rows: 16.2 us against 19.6).
+  // Two products would be two such launches and a second pass over grad_x
+  // (2816 x 1024, 8 experts, 5003 rows: the step of 669 us takes 30 more).
+  if (!pair && !tall_tiles(row_tiles(rows, E, 256) * ceil_div(K, TR_N)) && rows >= 96 * E) return false;
   return N % TR_K == 0 && K % 8 == 0 && K >= 192 && N <= (1 << 22) && K <= (1 << 22) &&
          (ceil_div(rows, 128) + E + kXcds) * ceil_div(K, TR_N) <= INT32_MAX / 8 && aligned(gy) && aligned(w) &&
          aligned(gx);
@@ -327,8 +338,7 @@ int gemm_tr_dx(const void* gy0, const void* gy1, const void* w0, const void* w1,
   a.experts = static_cast<int>(E);
   a.parts = gy1 ? 2 : 1;
   const int64_t nt = ceil_div(K, TR_N);
-  // on average half a row tile per expert is a remainder
-  const bool tall = tall_tiles((rows / 256.0 + 0.5 * E) * nt, (rows / 128.0 + 0.5 * E) * nt);
+  const bool tall = tall_tiles(row_tiles(rows, E, 256) * nt);
   const int64_t blocks = kXcds * nt * ceil_div(ceil_div(rows, tall ? 256 : 128) + E, kXcds);
   auto go = [&](auto dt, auto bt) {
     return tall ? launch_tr<decltype(dt)::value, 8, false, decltype(bt)::value, false>(a, blocks, stream)
@@ -362,8 +372,7 @@ int gemm_tr_dw(const void* gy0, const void* gy1, const void* x, int dtype, int64
   a.experts = static_cast<int>(E);
   a.parts = gy1 ? 2 : 1;
   const int64_t nt = ceil_div(K, TR_N), per = a.parts * E;
-  const bool tall = tall_tiles(static_cast<double>(per * nt * ceil_div(N, 256)),
-                               static_cast<double>(per * nt * ceil_div(N, 128)));
+  const bool tall = tall_tiles(static_cast<double>(per * nt * ceil_div(N, 256)));
   const int64_t blocks = kXcds * per * ceil_div(nt * ceil_div(N, tall ? 256 : 128), kXcds);
   auto go = [&](auto dt, auto c32) {
     return tall ? launch_tr<decltype(dt)::value, 8, true, false, decltype(c32)::value>(a, blocks, stream)

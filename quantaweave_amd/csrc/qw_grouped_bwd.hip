@@ -320,7 +320,8 @@ int gemm_grouped_backward(const void* gy, const void* x, const void* w, int dtyp
                           const int32_t* offsets, int64_t rows, int64_t rows_per_expert, void* gx, int accumulate,
                           void* gw, int gw_f32, bool tiled, void* ws, size_t ws_bytes, hipStream_t stream);
 
-bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows);
+bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows,
+                     bool pair);
 int gemm_tr_dx(const void* gy0, const void* gy1, const void* w0, const void* w1, int dtype, bool tiled, int64_t E,
                int64_t N, int64_t K, const int32_t* offsets, int64_t rows, void* gx, hipStream_t stream);
 bool gemm_tr_dw_fits(const void* gy, const void* x, const void* gw, int64_t E, int64_t N, int64_t K);
@@ -351,7 +352,7 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   const int64_t per = max_rows_per_expert > 0 && max_rows_per_expert < rows ? max_rows_per_expert : rows;
   QW_REQUIRE(ceil_div(per, BT) <= 65535 && ceil_div(N, BT) <= 65535, "grouped backward sizes out of range");
   // 256-column tiles over the operands as they lie (no workspace)
-  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && gemm_tr_dx_fits(gy, w, gx, E, N, K, rows)) {
+  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && gemm_tr_dx_fits(gy, w, gx, E, N, K, rows, false)) {
     const int st = gemm_tr_dx(gy, nullptr, w, nullptr, dtype, tiled, E, N, K, offsets, rows, gx, stream);
     if (st) return st;
     gx = nullptr;
@@ -429,8 +430,8 @@ int grouped_matmul_backward_pair(const void* gy_a, const void* gy_b, const void*
   if (gx != nullptr && rows > 0) QW_REQUIRE(gy_a && gy_b && w_a && w_b, "grad_x needs grad_out and w");
   if (gw_a != nullptr || gw_b != nullptr) QW_REQUIRE(rows == 0 || (gy_a && gy_b && x), "grad_w needs grad_out and x");
   // one accumulator for both: one rounding instead of two, and grad_x written once
-  if (is_half(dtype) && gx != nullptr && rows > 0 && gemm_tr_dx_fits(gy_a, w_a, gx, E, N, K, rows) &&
-      gemm_tr_dx_fits(gy_b, w_b, gx, E, N, K, rows)) {
+  if (is_half(dtype) && gx != nullptr && rows > 0 && gemm_tr_dx_fits(gy_a, w_a, gx, E, N, K, rows, true) &&
+      gemm_tr_dx_fits(gy_b, w_b, gx, E, N, K, rows, true)) {
     st = gemm_tr_dx(gy_a, gy_b, w_a, w_b, dtype, wfmt != dtype, E, N, K, offsets, rows, gx, stream);
     if (st) return st;
     gx = nullptr;

@@ -10,7 +10,11 @@ from quantaweave_amd import _hip, _lib, moe
 pytestmark = pytest.mark.gpu
 
 # rows per expert: none, one, around a 64-row slice, around both tile heights
-COUNTS = [[0, 1, 63, 64, 65, 129, 0, 257], [700], [5] * 40]
+UNEVEN = [0, 1, 63, 64, 65, 129, 0, 257]
+SIZES = [(128, 192), (64, 264), (96, 200), (320, 576), (1408, 512)]
+# the last three: enough tiles for the 256-row ones
+CASES = [(c, *nk) for c in (UNEVEN, [700], [5] * 40) for nk in SIZES] + [
+    (UNEVEN * 10, 128, 1024), (UNEVEN * 10, 64, 1000), (UNEVEN * 4 + [1], 576, 2816)]
 
 
 def check(got, want, bound, dtype):
@@ -40,8 +44,7 @@ def products(gys, x, ws, starts, counts):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("counts", COUNTS)
-@pytest.mark.parametrize("N,K", [(128, 192), (64, 264), (96, 200), (320, 576), (1408, 512)])
+@pytest.mark.parametrize("counts,N,K", CASES, ids=lambda v: str(len(v)) if isinstance(v, list) else str(v))
 def test_backward_on_operands_as_they_lie(dtype, counts, N, K):
     torch.manual_seed(N + K + len(counts))
     E, R, code = len(counts), sum(counts), _hip.HALF[dtype][0]
@@ -72,8 +75,8 @@ def test_backward_on_operands_as_they_lie(dtype, counts, N, K):
             _lib.call("qw_grouped_matmul_backward_pair", _hip.ptr(gys[0]), _hip.ptr(gys[1]), _hip.ptr(x),
                       _hip.ptr(weights[0]), _hip.ptr(weights[1]), code, fmt, *tail, _hip.ptr(gw[1]), _hip.ptr(gw[2]),
                       *end)
-            # off the tiles (N % 64) the first product is rounded before the second is added
-            check(gx, two[0], two[1] + (2.0 ** -8 * one[0].abs() if N % 64 else 0.0), dtype)
+            # as two products the first is rounded before the second is added
+            check(gx, two[0], two[1] + 2.0 ** -8 * one[0].abs(), dtype)
             for i in range(2):
                 check(gw[1 + i], two[2][i], two[3][i], out)
             assert torch.equal(gw[0], gw[1])
