@@ -11,13 +11,13 @@
 // projections' input gradients of a SwiGLU expert in place.
 //
 // bf16 and fp16 with a workspace run on the matrix cores (gemm_grouped_backward,
-// qw_gemm_mfma.hip); fp32 runs on the fp32 matrix cores (v_mfma_f32_16x16x4_f32,
-// the two kernels below) when rows are 16-byte aligned.  Otherwise two
+// qw_gemm_mfma.hip, or gemm_tr_dx and gemm_tr_dw, qw_gemm_tr.hip); fp32 runs on
+// the fp32 matrix cores (grouped_f32_kernel below) when rows are 16-byte aligned.  Otherwise two
 // vector-ALU kernels compute a 64x64 output tile per 256-thread
 // block (4x4 per thread) from 16-deep slices of the reduction staged in LDS;
 // the reduction runs in ascending order, so results do not depend on
 // scheduling.
-#include "qw_common.h"
+#include "qw_mfma.h"
 
 namespace qw {
 
@@ -128,74 +128,75 @@ __global__ __launch_bounds__(256) void grouped_dw_kernel(const void* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// fp32 on the matrix cores.  A 256-thread workgroup (2 x 2 waves) computes a
-// 64 x 64 output tile from 64-deep reduction slices staged in LDS (two
-// buffers; the next slice is loaded into registers while the current one is
-// multiplied).  Each LDS tile is [64 tile rows][64 reduction indices] with
-// the reduction contiguous, so a lane reads the 4 reduction values of a
-// 16-wide step with one 16-byte read; lane group q of the four 16x16x4
-// instructions of a step takes reduction index 4q + j (any assignment works
-// when both operands agree).  Operands whose reduction index is not the
-// contiguous one in memory are transposed on their way into LDS.  The
-// reduction runs in ascending order.
+// fp32 on the matrix cores (v_mfma_f32_16x16x4_f32, one fp32 per lane and
+// operand: lane group q of the four instructions j of a 16-wide step takes
+// reduction index 4q + j).  A 256-thread workgroup (2 x 2 waves) computes a
+// 64 x 64 output tile.  The matrix cores bound it (32 clocks an instruction), as
+// long as nothing waits: operands go straight to LDS (global_load_lds, a ring
+// of four 32-deep slices, three requested ahead) as they lie in memory.  A
+// reduction-major one is read one fp32 per lane, 16 columns of 4 rows: the
+// 16-column group c of row r sits at c ^ ((r / 4) % 4), so the four rows
+// cover all banks.  The other kind (rows of gy for grad_x) is read 16 bytes
+// per lane.  Transposing on the way into LDS, through registers, cost as many
+// LDS clocks as the products: F32_FIGURES.
+// The reduction runs in ascending order.
 // ---------------------------------------------------------------------------
 typedef float bf32x4 __attribute__((ext_vector_type(4)));
-constexpr int FB_T = 64, FB_R = 64, FB_LD = FB_R + 4;
+constexpr int FB_T = 64, FB_R = 32, FB_ST = 4, FB_OPER = FB_T * FB_R;  // tile, slice, stages, floats per operand
 
-// Products of one slice: acc[i][t] += A rows (wn*32 + 16t) x B rows (wm*32 + 16i)
-__device__ __forceinline__ void fb_compute(const float* As, const float* Bs, int wm, int wn, int l16, int lq,
-                                           bf32x4 (&acc)[2][2]) {
-#pragma unroll
-  for (int kk = 0; kk < FB_R; kk += 16) {
-    bf32x4 a[2], b[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) a[t] = *reinterpret_cast<const bf32x4*>(As + (wn * 32 + 16 * t + l16) * FB_LD + kk + 4 * lq);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) b[i] = *reinterpret_cast<const bf32x4*>(Bs + (wm * 32 + 16 * i + l16) * FB_LD + kk + 4 * lq);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], b[i][j], acc[i][t], 0, 0, 0);
-  }
-}
+__device__ const uint4 g_fb_zero = {0u, 0u, 0u, 0u};  // pieces past the end of the reduction
 
-// grad_x[r, k] (+)= sum_n gy[r, n] W_e[n, k]; block (k tile, row tile, expert).
-// A = W_e transposed into LDS ([k][n]), B = gy rows ([r][n]).
-__global__ __launch_bounds__(256) void grouped_dx_f32_kernel(const float* __restrict__ gy, const float* __restrict__ w,
-                                                             const int32_t* __restrict__ offsets, int N, int K,
-                                                             int rows, int accumulate, float* __restrict__ gx) {
-  __shared__ __attribute__((aligned(16))) float As[2][FB_T * FB_LD];
-  __shared__ __attribute__((aligned(16))) float Bs[2][FB_T * FB_LD];
+// RED: grad_W_e[n, k] = sum over the rows r of expert e of gy[r, n] a[r, k], a = x
+//      (exactly zero without rows); block (k tile, n tile, expert).
+// else: grad_x[r, k] (+)= sum_n gy[r, n] a[n, k], a = W_e; block (k tile, row tile, expert).
+template <bool RED>
+__global__ __launch_bounds__(256) void grouped_f32_kernel(const float* __restrict__ gy, const float* __restrict__ a,
+                                                          const int32_t* __restrict__ offsets, int N, int K, int rows,
+                                                          int accumulate, float* __restrict__ out) {
+  __shared__ __attribute__((aligned(1024))) float ring[FB_ST][2][FB_OPER];
   const int e = blockIdx.z;
   const int lo = min(max(offsets[e], 0), rows), hi = min(offsets[e + 1], rows);
-  const int r0 = lo + blockIdx.y * FB_T;
-  if (r0 >= hi) return;
-  const int k0 = blockIdx.x * FB_T;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int m0 = blockIdx.y * FB_T, k0 = blockIdx.x * FB_T;  // first row of the tile (of the expert's), first column
+  const int mcount = min(FB_T, (RED ? N : hi - lo) - m0);
+  if (mcount <= 0) return;
+  const int red = RED ? max(hi - lo, 0) : N;
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int wm = wave / 2, wn = wave % 2, l16 = lane % 16, lq = lane / 16;
-  const float* we = w + static_cast<int64_t>(e) * N * K;
-  // this thread's 16-byte pieces: tile rows tid/16 + 16h, columns 4*(tid%16)
-  const int pr = tid / 16, pc = 4 * (tid % 16);
-  bf32x4 ra[4], rb[4];
-  auto load = [&](int n0) {
+  // this lane's piece of load group wave + 4 q (1 KiB): source at the first
+  // slice, and the first reduction index it holds
+  const float *a_src[2], *b_src[2];
+  int a_red[2], b_red[2];
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const int n = n0 + pr + 16 * h, k = k0 + pc;  // W row n, columns k..k+3
-      ra[h] = (n < N && k < K) ? *reinterpret_cast<const bf32x4*>(we + static_cast<int64_t>(n) * K + k)
-                               : bf32x4{0.f, 0.f, 0.f, 0.f};
-      const int r = r0 + pr + 16 * h, nn = n0 + pc;  // gy row r, columns nn..nn+3
-      rb[h] = (r < hi && nn < N) ? *reinterpret_cast<const bf32x4*>(gy + static_cast<int64_t>(r) * N + nn)
-                                 : bf32x4{0.f, 0.f, 0.f, 0.f};
+  for (int q = 0; q < 2; ++q) {
+    const int g = wave + 4 * q;
+    const int r = 4 * g + lane / 16, c = 4 * ((lane % 16) ^ ((g & 3) << 2));
+    a_red[q] = r;
+    a_src[q] = a + (RED ? static_cast<int64_t>(lo) : static_cast<int64_t>(e) * N) * K + static_cast<int64_t>(r) * K +
+               min(k0 + c, K - 4);
+    if constexpr (RED) {
+      b_red[q] = r;
+      b_src[q] = gy + static_cast<int64_t>(lo + r) * N + min(m0 + c, N - 4);
+    } else {
+      const int row = 8 * g + lane / 8;
+      b_red[q] = 4 * ((lane % 8) ^ ((row >> 1) & 7));
+      b_src[q] = gy + static_cast<int64_t>(lo + m0 + min(row, mcount - 1)) * N + b_red[q];
     }
-  };
-  auto store = [&](int buf) {
+  }
+  const int64_t a_step = static_cast<int64_t>(FB_R) * K, b_step = RED ? static_cast<int64_t>(FB_R) * N : FB_R;
+  auto issue = [&](int s) {
+    float* st = &ring[s % FB_ST][0][0];
+    const int left = red - s * FB_R;  // reduction indices from this slice on
+    const float* zero = reinterpret_cast<const float*>(&g_fb_zero);
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
+    for (int q = 0; q < 2; ++q) {
+      const float* src = a_red[q] < left ? a_src[q] + s * a_step : zero;
+      __builtin_amdgcn_global_load_lds(static_cast<const void*>(src), (lds_void*)(st + (wave + 4 * q) * 256), 16, 0, 0);
+    }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) As[buf][(pc + j) * FB_LD + pr + 16 * h] = ra[h][j];  // [k][n]
-      *reinterpret_cast<bf32x4*>(&Bs[buf][(pr + 16 * h) * FB_LD + pc]) = rb[h];      // [r][n]
+    for (int q = 0; q < 2; ++q) {
+      const float* src = b_red[q] < left ? b_src[q] + s * b_step : zero;
+      __builtin_amdgcn_global_load_lds(static_cast<const void*>(src), (lds_void*)(st + FB_OPER + (wave + 4 * q) * 256),
+                                       16, 0, 0);
     }
   };
   bf32x4 acc[2][2];
@@ -203,111 +204,64 @@ __global__ __launch_bounds__(256) void grouped_dx_f32_kernel(const float* __rest
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int t = 0; t < 2; ++t) acc[i][t] = bf32x4{0.f, 0.f, 0.f, 0.f};
-  const int S = (N + FB_R - 1) / FB_R;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int sl = 0; sl < S; ++sl) {
-    if (sl + 1 < S) load((sl + 1) * FB_R);
-    fb_compute(As[sl & 1], Bs[sl & 1], wm, wn, l16, lq, acc);
-    if (sl + 1 < S) store((sl + 1) & 1);
-    __syncthreads();
-  }
-  // lane holds grad_x[row wm*32 + 16i + l16][k wn*32 + 16t + 4lq .. +3]
+  const int S = (red + FB_R - 1) / FB_R;  // 0 for an expert without rows
+  for (int s = 0; s < FB_ST - 1 && s < S; ++s) issue(s);
+  static_assert(FB_ST == 4, "the waits below");
+  for (int s = 0; s < S; ++s) {
+    // four loads per wave and slice; the two slices after this one stay in flight
+    if (s + 2 < S) wait_vmcnt<8>();
+    else if (s + 1 < S) wait_vmcnt<4>();
+    else wait_vmcnt<0>();
+    ring_barrier();
+    if (s + FB_ST - 1 < S) issue(s + FB_ST - 1);  // into the stage of slice s - 1
+    const float* As = &ring[s % FB_ST][0][0];
+    const float* Bs = As + FB_OPER;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = r0 + wm * 32 + 16 * i + l16;
-    if (r >= hi) continue;
+    for (int kk = 0; kk < FB_R; kk += 16) {
+      float av[2][4], bv[2][4];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int k = k0 + wn * 32 + 16 * t + 4 * lq;
-      float* o = gx + static_cast<int64_t>(r) * K + k;
-      if (k + 3 < K) {
-        bf32x4 v = acc[i][t];
-        if (accumulate) {
-          const bf32x4 old = *reinterpret_cast<const bf32x4*>(o);
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = old[j] + v[j];
+        for (int j = 0; j < 4; ++j) av[t][j] = As[(kk + 4 * lq + j) * FB_T + (((2 * wn + t) ^ lq) << 4) + l16];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (RED) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bv[i][j] = Bs[(kk + 4 * lq + j) * FB_T + (((2 * wm + i) ^ lq) << 4) + l16];
+        } else {
+          const int row = wm * 32 + 16 * i + l16;
+          const bf32x4 v = *reinterpret_cast<const bf32x4*>(Bs + row * FB_R + 4 * ((kk / 4 + lq) ^ ((row >> 1) & 7)));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bv[i][j] = v[j];
         }
-        *reinterpret_cast<bf32x4*>(o) = v;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (k + j < K) o[j] = accumulate ? o[j] + acc[i][t][j] : acc[i][t][j];
       }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[t][j], bv[i][j], acc[i][t], 0, 0, 0);
     }
   }
-}
-
-// grad_W_e[n, k] = sum over the rows r of expert e of gy[r, n] x[r, k] (exactly
-// zero without rows); block (k tile, n tile, expert).  A = x transposed
-// ([k][r]), B = gy transposed ([n][r]).
-__global__ __launch_bounds__(256) void grouped_dw_f32_kernel(const float* __restrict__ gy, const float* __restrict__ x,
-                                                             const int32_t* __restrict__ offsets, int N, int K,
-                                                             int rows, float* __restrict__ gw) {
-  __shared__ __attribute__((aligned(16))) float As[2][FB_T * FB_LD];
-  __shared__ __attribute__((aligned(16))) float Bs[2][FB_T * FB_LD];
-  const int e = blockIdx.z;
-  const int lo = min(max(offsets[e], 0), rows), hi = min(offsets[e + 1], rows);
-  const int n0 = blockIdx.y * FB_T, k0 = blockIdx.x * FB_T;
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int wm = wave / 2, wn = wave % 2, l16 = lane % 16, lq = lane / 16;
-  const int pr = tid / 16, pc = 4 * (tid % 16);
-  bf32x4 ra[4], rb[4];
-  auto load = [&](int m0) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const int r = m0 + pr + 16 * h;
-      const bool ok = r < hi;
-      ra[h] = (ok && k0 + pc < K) ? *reinterpret_cast<const bf32x4*>(x + static_cast<int64_t>(r) * K + k0 + pc)
-                                  : bf32x4{0.f, 0.f, 0.f, 0.f};
-      rb[h] = (ok && n0 + pc < N) ? *reinterpret_cast<const bf32x4*>(gy + static_cast<int64_t>(r) * N + n0 + pc)
-                                  : bf32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        As[buf][(pc + j) * FB_LD + pr + 16 * h] = ra[h][j];  // [k][r]
-        Bs[buf][(pc + j) * FB_LD + pr + 16 * h] = rb[h][j];  // [n][r]
-      }
-  };
-  bf32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) acc[i][t] = bf32x4{0.f, 0.f, 0.f, 0.f};
-  const int S = (hi - lo + FB_R - 1) / FB_R;  // 0 for an expert without rows
-  if (S > 0) {
-    load(lo);
-    store(0);
-  }
-  __syncthreads();
-  for (int sl = 0; sl < S; ++sl) {
-    if (sl + 1 < S) load(lo + (sl + 1) * FB_R);
-    fb_compute(As[sl & 1], Bs[sl & 1], wm, wn, l16, lq, acc);
-    if (sl + 1 < S) store((sl + 1) & 1);
-    __syncthreads();
-  }
-  // lane holds grad_W[n wm*32 + 16i + l16][k wn*32 + 16t + 4lq .. +3]
-  float* ge = gw + static_cast<int64_t>(e) * N * K;
+  // lane holds row wm*32 + 16i + l16, columns wn*32 + 16t + 4lq .. +3
+  float* const base = out + (RED ? static_cast<int64_t>(e) * N + m0 : static_cast<int64_t>(lo) + m0) * K;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int n = n0 + wm * 32 + 16 * i + l16;
-    if (n >= N) continue;
+    const int m = wm * 32 + 16 * i + l16;
+    if (m >= mcount) continue;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int k = k0 + wn * 32 + 16 * t + 4 * lq;
-      float* o = ge + static_cast<int64_t>(n) * K + k;
-      if (k + 3 < K) {
-        *reinterpret_cast<bf32x4*>(o) = acc[i][t];
-      } else {
+      if (k >= K) continue;  // K % 4 == 0: wholly inside or past the end
+      bf32x4* o = reinterpret_cast<bf32x4*>(base + static_cast<int64_t>(m) * K + k);
+      bf32x4 v = acc[i][t];
+      if (!RED && accumulate) {
+        const bf32x4 old = *o;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (k + j < K) o[j] = acc[i][t][j];
+        for (int j = 0; j < 4; ++j) v[j] = old[j] + v[j];
       }
+      *o = v;
     }
   }
 }
@@ -351,8 +305,11 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   if (gw != nullptr) QW_REQUIRE(rows == 0 || (gy && x), "grad_w needs grad_out and x");
   const int64_t per = max_rows_per_expert > 0 && max_rows_per_expert < rows ? max_rows_per_expert : rows;
   QW_REQUIRE(ceil_div(per, BT) <= 65535 && ceil_div(N, BT) <= 65535, "grouped backward sizes out of range");
-  // 256-column tiles over the operands as they lie (no workspace)
-  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && gemm_tr_dx_fits(gy, w, gx, E, N, K, rows, false)) {
+  // 256-column tiles over the operands as they lie (no workspace used; tiled
+  // weights without one stay refused, below)
+  const bool roomy = ws != nullptr && ws_bytes >= gemm_backward_workspace_bytes(E, N, K, rows);
+  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && (!tiled || roomy) &&
+      gemm_tr_dx_fits(gy, w, gx, E, N, K, rows, false)) {
     const int st = gemm_tr_dx(gy, nullptr, w, nullptr, dtype, tiled, E, N, K, offsets, rows, gx, stream);
     if (st) return st;
     gx = nullptr;
@@ -363,8 +320,7 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
     gw = nullptr;
   }
   // matrix-core path (bf16/fp16 with a workspace): dX needs out_features % 64 == 0, dW any shape
-  const bool core = is_half(dtype) && ws != nullptr && ws_bytes >= gemm_backward_workspace_bytes(E, N, K, rows) &&
-                    aligned16(gy) && aligned16(x) && aligned16(w) && gemm_backward_fits(rows, E);
+  const bool core = is_half(dtype) && roomy && aligned16(gy) && aligned16(x) && aligned16(w) && gemm_backward_fits(rows, E);
   const bool core_dx = core && gx != nullptr && aligned16(gx) && N % 64 == 0 && K % 4 == 0;
   const bool core_dw = core && gw != nullptr && aligned16(gw);
   if (core_dx || core_dw) {
@@ -383,17 +339,17 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   if (f32_core && gx != nullptr && rows > 0) {
     const dim3 g(static_cast<unsigned>(ceil_div(K, FB_T)), static_cast<unsigned>(ceil_div(per, FB_T)),
                  static_cast<unsigned>(E));
-    grouped_dx_f32_kernel<<<g, 256, 0, stream>>>(static_cast<const float*>(gy), static_cast<const float*>(w), offsets,
-                                                 n, k, r, accumulate, static_cast<float*>(gx));
-    QW_LAUNCH_CHECK("grouped_dx_f32_kernel");
+    grouped_f32_kernel<false><<<g, 256, 0, stream>>>(static_cast<const float*>(gy), static_cast<const float*>(w),
+                                                     offsets, n, k, r, accumulate, static_cast<float*>(gx));
+    QW_LAUNCH_CHECK("grouped_f32_kernel");
     gx = nullptr;
   }
   if (f32_core && gw != nullptr && gw_dtype == QW_F32) {
     const dim3 g(static_cast<unsigned>(ceil_div(K, FB_T)), static_cast<unsigned>(ceil_div(N, FB_T)),
                  static_cast<unsigned>(E));
-    grouped_dw_f32_kernel<<<g, 256, 0, stream>>>(static_cast<const float*>(gy), static_cast<const float*>(x), offsets,
-                                                 n, k, r, static_cast<float*>(gw));
-    QW_LAUNCH_CHECK("grouped_dw_f32_kernel");
+    grouped_f32_kernel<true><<<g, 256, 0, stream>>>(static_cast<const float*>(gy), static_cast<const float*>(x),
+                                                    offsets, n, k, r, 0, static_cast<float*>(gw));
+    QW_LAUNCH_CHECK("grouped_f32_kernel");
     gw = nullptr;
   }
   if (gx != nullptr && rows > 0) {

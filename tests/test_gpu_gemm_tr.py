@@ -96,3 +96,26 @@ def test_rows_past_an_expert_stay_out():
               _hip.ptr(offsets), 128, 0, None, 0, _hip.ptr(gw), _lib.QW_F32, None, 0, _hip.stream(x.device))
     g = gy[:70].double().t().contiguous()
     check(gw[0], g @ x[:70].double(), (g.abs() @ x[:70].double().abs()) * 134 * 2.0 ** -24, torch.float32)
+
+
+@pytest.mark.parametrize("counts,N,K", [(UNEVEN, 64, 64), (UNEVEN, 68, 132), (UNEVEN, 4, 8), ([700], 100, 64),
+                                        ([31, 32, 33], 128, 68)])
+def test_fp32_backward_on_operands_as_they_lie(counts, N, K):
+    """Slices of 32 and tiles of 64 with remainders in every direction, rows past an expert not finite."""
+    torch.manual_seed(N + K)
+    counts, E = [*counts, 9], len(counts) + 1
+    starts, R = [0, *torch.tensor(counts).cumsum(0).tolist()], sum(counts)
+    offsets = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    x, gy = torch.randn(R, K, device="cuda"), torch.randn(R, N, device="cuda")
+    x[-9:], gy[-9:] = float("inf"), float("nan")
+    w = torch.randn(E, N, K, device="cuda") * 0.05
+    gx, gw = torch.ones(R, K, device="cuda"), torch.full((E, N, K), 3.0, device="cuda")
+    print(f"case fp32 {N}x{K} rows {R}", flush=True)
+    for accumulate in (0, 1):
+        _lib.call("qw_grouped_matmul_backward", _hip.ptr(gy), _hip.ptr(x), _hip.ptr(w), _lib.QW_F32, E, N, K,
+                  _hip.ptr(offsets), R, 0, _hip.ptr(gx), accumulate, _hip.ptr(gw), _lib.QW_F32, None, 0,
+                  _hip.stream(x.device))
+        live = R - 9
+        dx, bound, dws, bounds = products([gy[:live]], x[:live], [w], starts, counts[:-1])
+        check(gx[:live], dx * (1 + accumulate), bound * (1 + accumulate), torch.float32)
+        check(gw[:-1], dws[0], bounds[0], torch.float32)
