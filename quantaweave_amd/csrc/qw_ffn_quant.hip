@@ -148,6 +148,15 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
   constexpr int DW = qp_dwords<WF, KS>();      // code dwords per lane, tile and slice
   static_assert(DW == 4 || DW == 2, "16- or 8-byte code loads");
   static_assert(A_STAGE % 4096 == 0, "whole load groups per wave");
+  // When the codes of the slice after the next are requested.  At first, over a copy
+  // of the present ones, where the registers hold the copy.  With 96 rows (SUB 6)
+  // they do so for bf16 int4 only; elsewhere 4 to 46 registers went to scratch, for
+  // fp16 inside the loop, so there the codes are multiplied where they lie and
+  // requested behind the slice's last conversions (64 rows per expert, fp16: int4 d
+  // 4096, f 1408 383 -> 306 us, int8 d 2048, f 1024 156 -> 121; bf16 int8 124 -> 117).
+  // Smaller chunks spend less time on a slice and need the longer lead (18 rows,
+  // int4: 223 us against 241).
+  constexpr bool LATE = SUB >= 6 && (WF == QW_I8 || ACT == QW_F16);
   extern __shared__ __attribute__((aligned(1024))) char smem[];
 
   // ---- tile: 8 experts or more: expert e's tiles go to XCD e % 8, so its rows
@@ -263,18 +272,19 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
       // end those of the last one), so the count is fixed.
       wait_vmcnt<AL + BL>();
       ring_barrier();  // visible to every wave, and every wave is done with slice kt - 1
-      uint32_t cw[QP_NT][DW];
+      const int next = min(kt + 2, KT - 1);
+      const int nstage = stage == 0 ? 2 : stage - 1;
+      issue_a(next, nstage);
+      uint32_t copy[QP_NT][DW];
+      uint32_t (&cw)[QP_NT][DW] = LATE ? raw[BUF] : copy;
       float cs[QP_NT], s4[QP_NT][STEPS];
 #pragma unroll
       for (int t = 0; t < QP_NT; ++t) {
 #pragma unroll
-        for (int i = 0; i < DW; ++i) cw[t][i] = raw[BUF][t][i];
+        for (int i = 0; i < (LATE ? 0 : DW); ++i) copy[t][i] = raw[BUF][t][i];
         cs[t] = RS ? row_sc[t] : sc[BUF][t];
       }
-      const int next = min(kt + 2, KT - 1);
-      const int nstage = stage == 0 ? 2 : stage - 1;
-      issue_a(next, nstage);
-      load_b(next, raw[BUF], sc[BUF]);
+      if constexpr (!LATE) load_b(next, raw[BUF], sc[BUF]);
       exchange<WF, KS, RS>(cw, cs, s4);
       const char* st = smem + stage * A_STAGE;
       stage = stage == 2 ? 0 : stage + 1;
@@ -287,6 +297,11 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
         bf16x8 w[QP_NT];
 #pragma unroll
         for (int t = 0; t < QP_NT; ++t) w[t] = weight_operand<ACT, WF, DW>(cw[t], s, s4[t][s]);
+        if (LATE && s == STEPS - 1) {
+          if constexpr (WF == QW_I8) __builtin_amdgcn_sched_barrier(0);
+          load_b(next, raw[BUF], sc[BUF]);
+          if constexpr (WF == QW_I8 && ACT == QW_F16) __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
           const bf16x8 xr = read_a(i, s);
