@@ -35,6 +35,7 @@
 // kernel of this file (ffn_qmf_kernel), which keeps the same streaming scheme
 // but forms the dot products on the 4x4x4 matrix cores; the kernel above serves
 // bf16 / fp16 weights and longer quantised rows.
+#include <algorithm>
 #include <cmath>
 
 #include "qw_ffn.h"
@@ -1361,18 +1362,35 @@ int launch_fmt(const FfnArgs& a, hipStream_t stream) {
   }
 }
 
+// Whether experts of this many rows are streamed rather than multiplied in
+// tiles.  Quantised weights: the streaming kernels multiply the exact codes, the
+// matrix-core ones rounded weights, and take over only from 16 rows.  16-bit
+// weights at widths that are no multiples of 64 have no matrix-core kernel
+// (200 x 520, 12 experts of 8 rows: 18 us streamed, 73 on the general kernel; 1544
+// x 776, 16 experts of 15: 108 / 617).  Others: a streaming pass takes 4 rows of an
+// expert and reads all its weights; the matrix-core kernel reads them once
+// whatever the rows, but walks the K slices one after another in few
+// workgroups.  Few experts therefore stream longer than many.  The two sides are
+// fits, in us, to 2 to 15 rows, 1 to 184 experts and widths of 64 to 4096
+// (streamed / not: 2048 x 1024, 64 experts of 2 / 3 / 8 rows 128 / 117, 151 / 120,
+// 310 / 129, 8 experts of 3 / 4 / 8 23 / 35, 34 / 35, 52 / 35, one expert of 3 / 15
+// 10 / 32, 24 / 32; 256 x 512, 8 experts of 3 / 5 11.1 / 12.7, 14.0 / 12.3).  Rows
+// of more than four chunks per lane (widths above 2048) stream more slowly (3072 x
+// 768, 6 experts of 5 rows 51 / 43, 4096 x 1408, one expert of 15 65 / 55).
+bool streamed(const FfnArgs& a) {
+  if (quantized(a.wfmt) || a.d_model % 64 || a.d_ff % 64) return a.avg_rows < 16;
+  if (a.avg_rows < 3 || a.avg_rows >= 16) return a.avg_rows < 3;
+  const double widths = static_cast<double>(a.d_model + a.d_ff);
+  const double megabytes = 6e-6 * a.d_model * a.d_ff * a.experts * (a.avg_rows + 3) / 4;  // read in all passes
+  const double per_megabyte = std::max(a.d_model, a.d_ff) > 2048 ? 0.3 : 0.12;
+  return 1.5 * ceil_div(a.avg_rows, 4) + per_megabyte * megabytes < 0.0095 * widths - 4.0;
+}
+
 }  // namespace
 
 int launch_ffn_gemv(const FfnArgs& a, hipStream_t stream, bool* handled) {
   *handled = false;
-  // 16-bit weights: a pass takes 4 rows of an expert and reads all its weights,
-  // the matrix-core kernel reads them once whatever the rows (whole layer, 64
-  // experts, d 2048, f 1024, streamed against not: 70 / 95 us at 16 tokens, 135
-  // / 137 at 64 = 2 rows per expert, 180 / 150 at 96, 206 / 153 at 128, 405 /
-  // 159 at 333).  Quantised weights: the streaming kernels multiply the exact
-  // codes, the matrix-core ones rounded weights, and take over only where they
-  // always did.
-  if (!is_half(a.act) || a.avg_rows >= (quantized(a.wfmt) ? 16 : 3)) return QW_OK;
+  if (!is_half(a.act) || !streamed(a)) return QW_OK;
   const bool f16 = a.act == QW_F16;
   if ((a.save_gate || a.save_y) && quantized(a.wfmt)) return QW_OK;  // quantised experts do not train
   // the matrix-core decode kernel's grid has a row per pass of up to 4 routes:

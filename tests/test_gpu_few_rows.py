@@ -47,3 +47,29 @@ def test_few_rows_per_expert(D, F_, counts, dtype):
         y = hipcall.experts(x, offsets, FMT[dtype], gate, up, down, path=path)
         err = ((y.double() - ref).abs().max() / ref.abs().max()).item()
         assert err <= tol, (path, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,F_,counts,path", [
+    # widths that are no multiples of 64: no matrix-core kernel takes them
+    (200, 520, [3, 2, 0, 7, 4, 1], "stream"), (200, 520, [8] * 12, "stream"), (200, 520, [15, 14, 15], "stream"),
+    (520, 192, [9, 0, 5], "stream"), (192, 72, [3], "stream"), (200, 520, [16, 17], "generic"),
+    # few experts stream longer than many
+    (1024, 1024, [8], "stream"), (512, 1024, [3] * 8, "stream"), (512, 1024, [8] * 8, "mfma"),
+    (256, 512, [2, 4, 3], "stream"), (256, 512, [12] * 8, "mfma"), (64, 128, [3] * 4, "mfma"),
+])
+def test_kernel_family_of_few_rows(D, F_, counts, path, dtype):
+    """auto takes the family that is the faster one at the size (same bits as that
+    family), and its result is right."""
+    torch.manual_seed(D + F_ + len(counts))
+    E = len(counts)
+    make = lambda *s: (torch.randn(*s, device="cuda") * 0.05).to(dtype)  # noqa: E731
+    gate, up, down = make(E, F_, D), make(E, F_, D), make(E, D, F_)
+    x = torch.randn(sum(counts), D, device="cuda").to(dtype)
+    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32, device="cuda")
+    print(f"case {D}x{F_} {counts} {dtype} {path}", flush=True)
+    y = hipcall.experts(x, offsets, FMT[dtype], gate, up, down)
+    assert torch.equal(y, hipcall.experts(x, offsets, FMT[dtype], gate, up, down, path=path))
+    ref = reference(x, counts, gate, up, down)
+    tol = 4 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)  # as above
+    assert ((y.double() - ref).abs().max() / ref.abs().max()).item() <= tol
