@@ -13,7 +13,7 @@
 // operation written.
 #include <type_traits>
 
-#include "qw_common.h"
+#include "qw_balance.h"
 
 namespace qw {
 
@@ -724,6 +724,8 @@ static int launch_topk(const float* partial, int splits, float temperature, floa
 // ---------------------------------------------------------------------------
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallTokens = 64;       // tokens of the one-workgroup plan
+// It writes no partial sums of the balance loss: one chunk has to hold its tokens.
+static_assert(kSmallTokens <= kImpRows, "the balance loss of the one-workgroup plan sums the probabilities directly");
 constexpr int kSmallRouteTokens = 16;  // tokens it also routes (one per wave)
 constexpr int kSmallRoutes = 256;
 constexpr int kSmallLogits = 8192;  // T*E logits staged in LDS

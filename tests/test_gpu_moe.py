@@ -512,6 +512,55 @@ def test_balance_with_workspace_matches_float64_and_is_deterministic(T, E, K):
     assert outs[0][1].numpy().astype(np.float32) == bal_ref
 
 
+@pytest.mark.parametrize("E", [8, 64, 65, 184, 1024])
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 1025, 4097])
+def test_forward_balance_equals_the_stand_alone_kernels(T, E):
+    """qw_moe_forward_balance, whose balance loss rides on the plan and combine
+    launches, returns the bits of qw_moe_balance_ws on its own probabilities and
+    counts, for one chunk of tokens (no partial sums) and many; the overflow count
+    and the zero; every other output is qw_moe_forward's.  The workspace holds NaN
+    before, so a partial sum that nothing wrote shows."""
+    from quantaweave_amd import _hip, _lib
+
+    D, F_, K = 16, 16, 2
+    torch.manual_seed(T * 1025 + E)
+    make = lambda *s: torch.randn(*s, device="cuda") * 0.1  # noqa: E731
+    x, rw, gate, up, down = make(T, D), make(E, D), make(E, F_, D), make(E, F_, D), make(E, D, F_)
+    R, cap, lib = T * K, max(1, T * K // E), _lib.load()
+
+    def forward(balance):
+        i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")  # noqa: E731
+        f32 = lambda n: torch.full((n,), float("nan"), device="cuda")  # noqa: E731
+        o = dict(out=f32(T * D), probs=f32(T * E), idx=i32(R), w=f32(R), counts=i32(E), kept=i32(E), totals=i32(2),
+                 dt=i32(R), de=i32(R))
+        tail = dict(imp=f32(E), bal=f32(1), overflow=torch.full((1,), -7, dtype=torch.int64, device="cuda"),
+                    zero=f32(1)) if balance else {}
+        name = "qw_moe_forward_balance" if balance else "qw_moe_forward"
+        nb = getattr(lib, name + "_workspace_bytes")(T, D, E, K, F_, _lib.QW_F32)
+        ws = torch.full((nb // 4 + 1,), float("nan"), device="cuda")
+        P = _hip.ptr
+        _lib.call(name, P(x), _lib.QW_F32, T, D, P(rw), _lib.QW_F32, 1.0, None, E, K, cap, F_, _lib.QW_F32, 0, 0,
+                  P(gate), None, P(up), None, P(down), None, *map(P, o.values()), *map(P, tail.values()), P(ws), nb,
+                  _hip.stream(x.device))
+        torch.cuda.synchronize()
+        n = int(o["totals"][1])  # dropped entries written
+        o["dt"], o["de"] = o["dt"][:n], o["de"][:n]
+        return {**o, **tail}
+
+    print(f"case T {T} E {E}", flush=True)
+    got, plain = forward(True), forward(False)
+    for name, t in plain.items():
+        assert torch.equal(got[name], t), name
+    nb = lib.qw_moe_balance_workspace_bytes(T, E)
+    ws = torch.full((max(nb // 4, 1),), float("nan"), device="cuda")
+    imp, bal = torch.empty(E, device="cuda"), torch.empty(1, device="cuda")
+    _lib.call("qw_moe_balance_ws", _hip.ptr(got["probs"]), _hip.ptr(got["counts"]), T, K, E, _hip.ptr(imp),
+              _hip.ptr(bal), _hip.ptr(ws), nb, _hip.stream(x.device))
+    assert torch.equal(got["imp"], imp) and torch.equal(got["bal"], bal)
+    assert torch.isfinite(got["bal"]).all()
+    assert int(got["overflow"]) == int(got["totals"][1]) and float(got["zero"]) == 0.0
+
+
 def _balance_fixed_order(probs, counts, T, K, E):
     """qw_moe_balance_ws's additions in order, in float32: per 64-token chunk
     four strided sums (tokens j, j + 4, ... of the chunk) added as ((s0 + s1) + s2)
