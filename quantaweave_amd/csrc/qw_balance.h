@@ -55,71 +55,92 @@ __device__ __forceinline__ void importance_unit(const BalanceJob& j, int unit, f
     j.partial[static_cast<int64_t>(chunk) * j.E + e] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
-// Sum w of expert e: partial rows w, w + 16, ... in order, eight in flight.
-__device__ __forceinline__ float importance_sum(const BalanceJob& j, int w, int e) {
-  constexpr int kRowsPerLoad = 8;
-  float s = 0.0f;
+// Sums w, w + 16 / NS, ... (NS of the sixteen) of expert e, sum i over the partial rows
+// i, i + 16, ... in order: eight rows of each in flight.  w is uniform: one row
+// address per wave and load.
+template <int NS>
+__device__ __forceinline__ void importance_sums(const BalanceJob& j, int w, int e, float (&s)[NS]) {
+  constexpr int kRows = 8, kStep = 16 / NS;
+  const int col = min(e, j.E - 1);
+#pragma unroll
+  for (int i = 0; i < NS; ++i) s[i] = 0.0f;
 #pragma unroll 1
-  for (int b0 = w; b0 < j.nb; b0 += 16 * kRowsPerLoad) {
-    float v[kRowsPerLoad];
+  for (int b0 = w; b0 < j.nb; b0 += 16 * kRows) {
+    float v[NS * kRows];
 #pragma unroll
-    for (int i = 0; i < kRowsPerLoad; ++i) {
-      const int b = b0 + 16 * i;
-      v[i] = (b < j.nb && e < j.E) ? j.partial[static_cast<int64_t>(b) * j.E + e] : 0.0f;
-    }
+    for (int k = 0; k < NS * kRows; ++k)  // rows past the end: the last one, not added
+      v[k] = (j.partial + static_cast<int64_t>(min(b0 + kStep * k, j.nb - 1)) * j.E)[col];
 #pragma unroll
-    for (int i = 0; i < kRowsPerLoad; ++i) s += v[i];  // rows in order; +0 past the end (sums are >= 0)
+    for (int k = 0; k < NS * kRows; ++k) s[k % NS] += b0 + kStep * k < j.nb ? v[k] : 0.0f;  // +0: sums are >= 0
   }
-  return s;
 }
 
-// Importance and balance by one 256-thread workgroup: sixteen sums per expert
-// (a single chunk: its four quarters, straight from the probabilities) added
-// in order, then the balance term over experts in ascending order by one
-// thread.  Up to 64 experts the sums are dealt over the four waves, beyond
-// that the blocks of 64 experts.  It runs beside the combining workgroups, so
-// it keeps few loads in flight: 32 took 138 registers per thread, which every
-// one of them paid for (combine 16 -> 24 us at 8192 x 2048).
+// Importance and balance by one workgroup of WAVES waves (4 or 16): sixteen sums per
+// expert (a single chunk: its four quarters, straight from the probabilities)
+// added in order, then the balance term over experts in ascending order by one
+// thread.  Bound by the rounds of dependent loads.  64 experts at a time, the sums
+// dealt over the waves: one round per 128 partial rows and 64 experts (184 experts:
+// 3 at 8192 tokens; a thread per expert, its sums one after the other, took 16: whole
+// layer of d 64, 71.7 -> 66.9 us, 1024 experts 201 -> 193).  With at most 16 partial
+// rows a sum is one row: a thread per expert then holds all of them in one round
+// (184 experts, 256 tokens: 37.8 us against 40.7).  With 4 waves it runs beside the
+// combining workgroups, which pay for its registers: 49 here, 138 with 64-bit
+// addresses per lane (combine 16 -> 24 us at 8192 x 2048).
+// A kernel of its own is built for one form (kThreadPerExpert: more than 64 experts
+// and at most 16 partial rows; kManyRows: several partial rows): its instructions
+// come from memory at each launch, and those of the other forms cost it 1 us.
+enum BalanceForm { kAnyForm, kThreadPerExpert, kManyRows };
+
+template <int WAVES, BalanceForm FORM = kAnyForm>
 __device__ __forceinline__ void balance_final(const BalanceJob& j, float (*red)[kWave], float* term) {
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  static_assert(WAVES == 4 || WAVES == 16, "sixteen sums dealt evenly, at least four quarters");
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const float routes = static_cast<float>(static_cast<int64_t>(j.T) * j.K);
-  const int sums = j.nb == 1 ? 4 : 16;
-  auto sum = [&](int w, int e) {
-    return j.nb == 1 ? importance_quarter(j.probs, j.T, j.E, 0, w, e) : importance_sum(j, w, e);
-  };
+  const bool one = FORM != kManyRows && j.nb == 1;
+  const int sums = one ? 4 : 16;
   auto finish = [&](float t, int e) {
     const float imp = t / static_cast<float>(j.T);
     j.importance[e] = imp;
     term[e] = imp * (static_cast<float>(j.counts[e]) / routes);
   };
-  if (j.E <= kWave) {
+  if (FORM == kThreadPerExpert || (FORM == kAnyForm && j.E > kWave && j.nb <= 16)) {
 #pragma unroll 1
-    for (int w = wave; w < sums; w += 4) red[w][lane] = sum(w, lane);
-    __syncthreads();
-    if (wave == 0 && lane < j.E) {
+    for (int e = threadIdx.x; e < j.E; e += WAVES * kWave) {
       float t = 0.0f;  // 0 + the first sum is that sum: all are >= 0
-      for (int w = 0; w < sums; ++w) t += red[w][lane];
-      finish(t, lane);
-    }
-  } else {
+      if (j.nb == 1) {
 #pragma unroll 1
-    for (int e = threadIdx.x; e - lane < j.E; e += 256) {
-      float t = 0.0f;
-      if (j.nb > 1 && j.nb <= 16) {  // one row per sum: all of them in flight
+        for (int q = 0; q < 4; ++q) t += importance_quarter(j.probs, j.T, j.E, 0, q, e);
+      } else {
         float v[16];
 #pragma unroll
-        for (int w = 0; w < 16; ++w)
-          v[w] = (w < j.nb && e < j.E) ? j.partial[static_cast<int64_t>(w) * j.E + e] : 0.0f;
+        for (int w = 0; w < 16; ++w) v[w] = (j.partial + static_cast<int64_t>(min(w, j.nb - 1)) * j.E)[e];
 #pragma unroll
-        for (int w = 0; w < 16; ++w) t += v[w];
-      } else {
-#pragma unroll 1
-        for (int w = 0; w < sums; ++w) t += sum(w, e);
+        for (int w = 0; w < 16; ++w) t += w < j.nb ? v[w] : 0.0f;
       }
-      if (e < j.E) finish(t, e);
+      finish(t, e);
+    }
+    __syncthreads();
+  } else {
+#pragma unroll 1
+    for (int e0 = 0; e0 < j.E; e0 += kWave) {
+      const int e = e0 + lane;
+      if (one) {
+        if (wave < 4) red[wave][lane] = importance_quarter(j.probs, j.T, j.E, 0, wave, e);
+      } else {
+        float s[16 / WAVES];
+        importance_sums<16 / WAVES>(j, wave, e, s);
+#pragma unroll
+        for (int i = 0; i < 16 / WAVES; ++i) red[wave + WAVES * i][lane] = s[i];
+      }
+      __syncthreads();
+      if (wave == 0 && e < j.E) {
+        float t = 0.0f;
+        for (int w = 0; w < sums; ++w) t += red[w][lane];
+        finish(t, e);
+      }
+      __syncthreads();
     }
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
     // ascending order; 16 reads in flight at a time (the terms are >= 0, so
     // the +0 past E changes nothing)

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const void* __restrict__ y
     __shared__ float red[16][kWave];
     __shared__ float term[1024];
     if (job.balance != nullptr && blockIdx.x == 0) {
-      balance_final(job, red, term);
+      balance_final<4>(job, red, term);
       return;
     }
   }
@@ -622,10 +622,13 @@ __global__ __launch_bounds__(256) void importance_partial_kernel(const BalanceJo
   importance_unit(job, blockIdx.x, red);
 }
 
-__global__ __launch_bounds__(256) void importance_final_kernel(const BalanceJob job) {
+// Alone on the chip it takes 16 waves (8192 tokens, 184 experts: 11.2 us with the
+// partial sums, 17.3 with 4 waves in all forms).
+template <int WAVES, BalanceForm FORM>
+__global__ __launch_bounds__(WAVES * kWave) void importance_final_kernel(const BalanceJob job) {
   __shared__ float red[16][kWave];
   __shared__ float term[1024];
-  balance_final(job, red, term);
+  balance_final<WAVES, FORM>(job, red, term);
 }
 
 size_t balance_workspace_bytes(int64_t T, int64_t E) {
@@ -653,7 +656,9 @@ int balance_ws(const float* probs, const int32_t* counts, int64_t T, int64_t K, 
     importance_partial_kernel<<<static_cast<unsigned>(partial_units(job.nb, job.E)), 256, 0, stream>>>(job);
     QW_LAUNCH_CHECK("importance_partial_kernel");
   }
-  importance_final_kernel<<<1, 256, 0, stream>>>(job);
+  if (job.nb <= 16 && E > kWave) importance_final_kernel<16, kThreadPerExpert><<<1, 1024, 0, stream>>>(job);
+  else if (job.nb > 1) importance_final_kernel<16, kManyRows><<<1, 1024, 0, stream>>>(job);
+  else importance_final_kernel<4, kAnyForm><<<1, 256, 0, stream>>>(job);
   QW_LAUNCH_CHECK("importance_final_kernel");
   return QW_OK;
 }

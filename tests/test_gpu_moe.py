@@ -513,7 +513,7 @@ def test_balance_with_workspace_matches_float64_and_is_deterministic(T, E, K):
 
 
 @pytest.mark.parametrize("E", [8, 64, 65, 184, 1024])
-@pytest.mark.parametrize("T", [1, 63, 64, 65, 1025, 4097])
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 1024, 1025, 4097, 8200])
 def test_forward_balance_equals_the_stand_alone_kernels(T, E):
     """qw_moe_forward_balance, whose balance loss rides on the plan and combine
     launches, returns the bits of qw_moe_balance_ws on its own probabilities and
