@@ -321,6 +321,9 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
   if (SUB >= 6 && active > 4) k_loop(std::integral_constant<int, SUB>{});
   else if (SUB >= 4 && active > 2) k_loop(std::integral_constant<int, SUB < 4 ? SUB : 4>{});
   else k_loop(std::integral_constant<int, 2>{});
+  // The last two slices asked for once too often still write to the stages, which
+  // the epilogue reuses and the workgroup's end gives back.
+  wait_vmcnt<0>();
 
   // ---- epilogue: lane holds row l16 of a sub-tile, columns 4 lq .. 4 lq + 3
   //      of each weight tile ----
