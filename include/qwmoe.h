@@ -390,7 +390,9 @@ int qw_grouped_matmul_backward(const void* grad_out, const void* x, const void* 
                                int grad_w_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same with the weights in w_format: `dtype`, or its tiles (QW_BF16T,
- * QW_F16T), which the matrix-core grad_x reads as they are. */
+ * QW_F16T), which the matrix-core grad_x reads as they are: without a workspace
+ * only where the 256-column tiles apply (else QW_ERR_UNSUPPORTED), in the pair
+ * below too. */
 int qw_grouped_matmul_backward_fmt(const void* grad_out, const void* x, const void* w, int dtype, int w_format,
                                    int64_t experts, int64_t out_features, int64_t in_features, const int32_t* offsets,
                                    int64_t rows, int64_t max_rows_per_expert, void* grad_x, int accumulate_grad_x,

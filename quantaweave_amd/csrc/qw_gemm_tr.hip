@@ -306,16 +306,19 @@ bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 
 }  // namespace
 
-// dX of one product, or of two summed (gy1, w1 non-null): N columns of gy are the reduction.
+// dX of one product, or of two summed (gy1, w1 non-null): N columns of gy are the
+// reduction.  tiles128: gemm_nt_kernel would take the product otherwise.
 bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows,
-                     bool pair) {
+                     bool pair, bool tiles128) {
   // One product: 128 x 128 tiles (gemm_nt_kernel) are level or faster where 256-row
   // tiles do not fill the chip (1024 x 2048, 16 experts, 4000 rows: 28.0 us against
   // 28.6; 512 x 256, 16000 rows: 14.4 against 15.7), except below 96 rows an
   // expert, where whole sub-tiles are skipped (1000 rows: 16.2 us against 19.6).
+  // They need a workspace; without one the product would go to the vector-ALU kernel
+  // (1024 x 512, 8 experts, 4000 rows: 174 us, 21 here).
   // Two products would be two such launches and a second pass over grad_x
   // (2816 x 1024, 8 experts, 5003 rows: the step of 669 us takes 30 more).
-  if (!pair && !tall_tiles(row_tiles(rows, E, 256) * ceil_div(K, TR_N)) && rows >= 96 * E) return false;
+  if (!pair && tiles128 && !tall_tiles(row_tiles(rows, E, 256) * ceil_div(K, TR_N)) && rows >= 96 * E) return false;
   return N % TR_K == 0 && K % 8 == 0 && K >= 192 && N <= (1 << 22) && K <= (1 << 22) &&
          (ceil_div(rows, 128) + E + kXcds) * ceil_div(K, TR_N) <= INT32_MAX / 8 && aligned(gy) && aligned(w) &&
          aligned(gx);

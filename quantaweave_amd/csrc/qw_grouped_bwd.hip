@@ -277,7 +277,7 @@ int gemm_grouped_backward(const void* gy, const void* x, const void* w, int dtyp
                           void* gw, int gw_f32, bool tiled, void* ws, size_t ws_bytes, hipStream_t stream);
 
 bool gemm_tr_dx_fits(const void* gy, const void* w, const void* gx, int64_t E, int64_t N, int64_t K, int64_t rows,
-                     bool pair);
+                     bool pair, bool tiles128);
 int gemm_tr_dx(const void* gy0, const void* gy1, const void* w0, const void* w1, int dtype, bool tiled, int64_t E,
                int64_t N, int64_t K, const int32_t* offsets, int64_t rows, void* gx, hipStream_t stream);
 bool gemm_tr_dw_fits(const void* gy, const void* x, const void* gw, int64_t E, int64_t N, int64_t K);
@@ -307,11 +307,14 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
   if (gw != nullptr) QW_REQUIRE(rows == 0 || (gy && x), "grad_w needs grad_out and x");
   const int64_t per = max_rows_per_expert > 0 && max_rows_per_expert < rows ? max_rows_per_expert : rows;
   QW_REQUIRE(ceil_div(per, BT) <= 65535 && ceil_div(N, BT) <= 65535, "grouped backward sizes out of range");
-  // 256-column tiles over the operands as they lie (no workspace used; tiled
-  // weights without one stay refused, below)
-  const bool roomy = ws != nullptr && ws_bytes >= gemm_backward_workspace_bytes(E, N, K, rows);
-  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 && (!tiled || roomy) &&
-      gemm_tr_dx_fits(gy, w, gx, E, N, K, rows, false)) {
+  // 128 x 128 tiles (bf16/fp16 with a workspace): dX needs out_features % 64 == 0, dW any shape
+  const bool core = is_half(dtype) && ws != nullptr && ws_bytes >= gemm_backward_workspace_bytes(E, N, K, rows) &&
+                    aligned16(gy) && aligned16(x) && aligned16(w) && gemm_backward_fits(rows, E);
+  const bool core_dx = core && aligned16(gx) && N % 64 == 0 && K % 4 == 0;
+  const bool core_dw = core && aligned16(gw);
+  // 256-column tiles over the operands as they lie (no workspace used)
+  if (is_half(dtype) && gx != nullptr && !accumulate && rows > 0 &&
+      gemm_tr_dx_fits(gy, w, gx, E, N, K, rows, false, core_dx)) {
     const int st = gemm_tr_dx(gy, nullptr, w, nullptr, dtype, tiled, E, N, K, offsets, rows, gx, stream);
     if (st) return st;
     gx = nullptr;
@@ -321,11 +324,7 @@ int grouped_matmul_backward(const void* gy, const void* x, const void* w, int dt
     if (st) return st;
     gw = nullptr;
   }
-  // matrix-core path (bf16/fp16 with a workspace): dX needs out_features % 64 == 0, dW any shape
-  const bool core = is_half(dtype) && roomy && aligned16(gy) && aligned16(x) && aligned16(w) && gemm_backward_fits(rows, E);
-  const bool core_dx = core && gx != nullptr && aligned16(gx) && N % 64 == 0 && K % 4 == 0;
-  const bool core_dw = core && gw != nullptr && aligned16(gw);
-  if (core_dx || core_dw) {
+  if ((core_dx && gx != nullptr) || (core_dw && gw != nullptr)) {
     const int st = gemm_grouped_backward(gy, x, w, dtype, E, N, K, offsets, rows, per, core_dx ? gx : nullptr, accumulate,
                                          core_dw ? gw : nullptr, gw_dtype == QW_F32, tiled, ws, ws_bytes, stream);
     if (st) return st;
@@ -388,8 +387,8 @@ int grouped_matmul_backward_pair(const void* gy_a, const void* gy_b, const void*
   if (gx != nullptr && rows > 0) QW_REQUIRE(gy_a && gy_b && w_a && w_b, "grad_x needs grad_out and w");
   if (gw_a != nullptr || gw_b != nullptr) QW_REQUIRE(rows == 0 || (gy_a && gy_b && x), "grad_w needs grad_out and x");
   // one accumulator for both: one rounding instead of two, and grad_x written once
-  if (is_half(dtype) && gx != nullptr && rows > 0 && gemm_tr_dx_fits(gy_a, w_a, gx, E, N, K, rows, true) &&
-      gemm_tr_dx_fits(gy_b, w_b, gx, E, N, K, rows, true)) {
+  if (is_half(dtype) && gx != nullptr && rows > 0 && gemm_tr_dx_fits(gy_a, w_a, gx, E, N, K, rows, true, false) &&
+      gemm_tr_dx_fits(gy_b, w_b, gx, E, N, K, rows, true, false)) {
     st = gemm_tr_dx(gy_a, gy_b, w_a, w_b, dtype, wfmt != dtype, E, N, K, offsets, rows, gx, stream);
     if (st) return st;
     gx = nullptr;

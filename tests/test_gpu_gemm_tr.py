@@ -119,3 +119,35 @@ def test_fp32_backward_on_operands_as_they_lie(counts, N, K):
         dx, bound, dws, bounds = products([gy[:live]], x[:live], [w], starts, counts[:-1])
         check(gx[:live], dx * (1 + accumulate), bound * (1 + accumulate), torch.float32)
         check(gw[:-1], dws[0], bounds[0], torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("E,N,K,rows", [(8, 128, 256, 1600), (3, 64, 192, 300), (2, 192, 264, 500)])
+def test_input_gradient_without_workspace(dtype, E, N, K, rows):
+    """At sizes where the 128 x 128 tiles are the preferred kernel, which need a
+    workspace: without one grad_x still runs on the 256-column tiles (the bits of a
+    pair whose second product is zero), plain weights and tiles alike."""
+    torch.manual_seed(N + K)
+    code, tile_code = _hip.HALF[dtype]
+    counts = [rows // E] * (E - 1) + [rows - rows // E * (E - 1)]
+    starts = [0, *torch.tensor(counts).cumsum(0).tolist()]
+    offsets = torch.tensor(starts, dtype=torch.int32, device="cuda")
+    gy = torch.randn(rows, N, device="cuda").to(dtype)
+    w = (torch.randn(E, N, K, device="cuda") * 0.05).to(dtype)
+    x = torch.empty(rows, K, dtype=dtype, device="cuda")  # read by the weight gradients only
+    want, bound, _, _ = products([gy], x.zero_(), [w], starts, counts)
+    zero = torch.zeros_like(gy)
+    formats = [(code, w)]
+    if N % 64 == 0 and K % 64 == 0:
+        formats.append((tile_code, moe.tile_bf16(w)))
+    for fmt, weights in formats:
+        print(f"case {N}x{K} {dtype} rows {rows} format {fmt}", flush=True)
+        gx, pair = (torch.full((rows, K), 3.0, dtype=dtype, device="cuda") for _ in range(2))
+        tail = (E, N, K, _hip.ptr(offsets), rows, 0)
+        _lib.call("qw_grouped_matmul_backward_fmt", _hip.ptr(gy), None, _hip.ptr(weights), code, fmt, *tail,
+                  _hip.ptr(gx), 0, None, code, None, 0, _hip.stream(gy.device))
+        _lib.call("qw_grouped_matmul_backward_pair", _hip.ptr(gy), _hip.ptr(zero), None, _hip.ptr(weights),
+                  _hip.ptr(weights), code, fmt, *tail, _hip.ptr(pair), None, None, code, None, 0,
+                  _hip.stream(gy.device))
+        check(gx, want, bound, dtype)
+        assert torch.equal(gx, pair)
