@@ -204,8 +204,6 @@ class ExpertPack:
         self._token = None
         if self.fmt in (_lib.QW_F32, _lib.QW_BF16, _lib.QW_F16):
             self.gate_s = self.up_s = self.down_s = None
-            self._float_weights = [[e._modules[n]._parameters["weight"].detach() for e in self._exps]
-                                   for n in ("gate", "up", "down")]
             if self.fmt != _lib.QW_F32:  # fp32 stacks are made on first use: 16-bit arithmetic reads only its copies
                 self._stack_float()
         else:
@@ -223,20 +221,27 @@ class ExpertPack:
                         m.qweight, m.scales = q[i], sc[i]
         self._record(experts)
 
-    def _tileable(self) -> bool:
+    def _float_weights(self) -> list:
+        """The float experts' own gate, up and down matrices.  Read from the modules
+        each time: a reference kept here would hold their storage after the modules
+        moved to another device or type."""
+        return [[e._modules[n]._parameters["weight"] for e in self._exps] for n in ("gate", "up", "down")]
+
+    @staticmethod
+    def _tileable(weights: list) -> bool:
         """The float experts' stacks can be tiles: all three projections, on a ROCm device."""
-        return all(w[0].device.type == "cuda" and w[0].size(0) % 64 == 0 and w[0].size(1) % 64 == 0
-                   for w in self._float_weights)
+        return all(w[0].device.type == "cuda" and w[0].size(0) % 64 == 0 and w[0].size(1) % 64 == 0 for w in weights)
 
     def _stack_float(self) -> None:
-        dt = self._float_weights[0][0].dtype
-        tile = dt in _hip.HALF and self._tileable()
-        self.gate, self.up, self.down = (pack_weights(w, dt, tile) for w in self._float_weights)
+        weights = self._float_weights()
+        dt = weights[0][0].dtype
+        tile = dt in _hip.HALF and self._tileable(weights)
+        self.gate, self.up, self.down = (pack_weights(w, dt, tile) for w in weights)
         if tile:
             self.fmt = _hip.HALF[dt][1]
 
     def __getattr__(self, name: str):
-        if name in ("gate", "up", "down") and "_float_weights" in self.__dict__:
+        if name in ("gate", "up", "down") and self.__dict__.get("_quant") is False:
             self._stack_float()
             return self.__dict__[name]
         raise AttributeError(name)
@@ -356,7 +361,7 @@ class ExpertPack:
             return src.fmt, stacks
         cache = self.__dict__.get("_plain")
         if cache is None or cache[0] != dtype:
-            cache = (dtype, [pack_weights(w, dtype, False) for w in self._float_weights])
+            cache = (dtype, [pack_weights(w, dtype, False) for w in self._float_weights()])
             self._plain = cache
         return code, cache[1]
 
@@ -381,8 +386,9 @@ class ExpertPack:
             cast = ExpertPack.__new__(ExpertPack)
             cast.fmt, cast.group_in, cast.group_ff = act, 0, 0
             cast.gate_s = cast.up_s = cast.down_s = None
+            weights = self._float_weights()
             # the masters, or a decode step's stacks moved to its device
-            if "gate" in self.__dict__ and self.gate.device != self._float_weights[0][0].device:
+            if "gate" in self.__dict__ and self.gate.device != weights[0][0].device:
                 # tiles are a permutation of the elements: a cast keeps them tiles
                 cast.gate, cast.up, cast.down = (t.to(dt).contiguous() for t in (self.gate, self.up, self.down))
                 if self.fmt in plain_of:
@@ -390,8 +396,8 @@ class ExpertPack:
                 else:
                     cast.maybe_tile()
             else:
-                tile = self._tileable()
-                cast.gate, cast.up, cast.down = (pack_weights(w, dt, tile) for w in self._float_weights)
+                tile = self._tileable(weights)
+                cast.gate, cast.up, cast.down = (pack_weights(w, dt, tile) for w in weights)
                 if tile:
                     cast.fmt = _hip.HALF[dt][1]
             copies[act] = cast

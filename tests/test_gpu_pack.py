@@ -5,6 +5,7 @@ torch operations (or the plain layout) it stands for."""
 import pytest
 import torch
 
+import quantaweave_amd as qa
 from quantaweave_amd import _hip, _lib, moe
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,22 @@ def test_gathered_rows_with_a_cast(src, dst, D):
               _hip.ptr(out), _hip.act_code(out, "out"), _hip.stream(x.device))
     assert torch.equal(out[:5], x.to(dst)[slots[:5].long()])
     assert (out[5] == 2.0).all()  # past the kept rows: untouched
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_pack_does_not_hold_the_experts_weights(dtype):
+    """A layer and a decode step keep their stacks, not the storage the stacks were
+    made from: moving the module frees it."""
+    config = qa.QuantaWeaveConfig(vocab_size=2, hidden_size=256, layers=1, ffn_size=512, num_experts=16, top_k=2,
+                                  attention_heads=1, max_sequence_length=64)
+    layer = qa.TopKMoE(config).to("cuda", dtype)
+    with torch.no_grad():
+        layer(torch.randn(1, 8, 256, device="cuda", dtype=dtype))
+    step = qa.MoEDecodeStep(layer, precision="bf16")
+    weights = sum(p.numel() * p.element_size() for p in layer.experts.parameters())
+    x = torch.randn(1, 256, device="cuda")
+    want = step.step(x).clone()
+    before = torch.cuda.memory_allocated()
+    layer.cpu()
+    assert before - torch.cuda.memory_allocated() >= weights
+    assert torch.equal(step.step(x), want)
