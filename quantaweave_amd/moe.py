@@ -201,6 +201,8 @@ class ExpertPack:
         self.fmt, self.group_in, self.group_ff = _expert_format(experts)
         self._exps = tuple(experts._modules.values())
         self._quant = isinstance(self._exps[0]._modules["gate"], QuantizedLinear)
+        gate = experts[0].gate
+        self.ffn = int((gate.qweight if self._quant else gate.weight).size(0))  # rows of the stored matrices
         self._token = None
         if self.fmt in (_lib.QW_F32, _lib.QW_BF16, _lib.QW_F16):
             self.gate_s = self.up_s = self.down_s = None
@@ -384,7 +386,7 @@ class ExpertPack:
         if act not in copies:
             dt = torch.bfloat16 if act == _lib.QW_BF16 else torch.float16
             cast = ExpertPack.__new__(ExpertPack)
-            cast.fmt, cast.group_in, cast.group_ff = act, 0, 0
+            cast.fmt, cast.group_in, cast.group_ff, cast.ffn = act, 0, 0, self.ffn
             cast.gate_s = cast.up_s = cast.down_s = None
             weights = self._float_weights()
             # the masters, or a decode step's stacks moved to its device
@@ -655,14 +657,13 @@ def _forward_call(flat: Tensor, act: int, router_w: Tensor, moe: TopKMoE, pack: 
         ints[:2 + R + 2 * E + 2].zero_()
         flts.zero_()
         return r
-    key = (T, width, E, K, act)
-    sizes = moe.__dict__.setdefault("_qw_sizes", {}).get(key)
+    d_ff = pack.ffn
+    sizes = moe.__dict__.setdefault("_qw_sizes", {})
+    key = (T, width, E, K, act, d_ff)
     lib = _lib.load()
-    if sizes is None:
-        d_ff = moe.experts[0].gate.out_features
-        sizes = (d_ff, lib.qw_moe_forward_balance_workspace_bytes(T, width, E, K, d_ff, act))
-        moe._qw_sizes[key] = sizes
-    d_ff, nbytes = sizes
+    nbytes = sizes.get(key)
+    if nbytes is None:
+        nbytes = sizes[key] = lib.qw_moe_forward_balance_workspace_bytes(T, width, E, K, d_ff, act)
     s = torch.cuda.current_stream(dev).cuda_stream
     wp = _stream_workspace(moe, nbytes, dev, s).data_ptr()
     ip, fp = ints.data_ptr() + 8, flts.data_ptr()  # top_idx, probs

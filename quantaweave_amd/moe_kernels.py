@@ -235,7 +235,7 @@ def grouped_swiglu(inputs: Tensor, experts: nn.ModuleList, counts: Sequence[int]
     # the reference casts the stacked weights to the compute dtype (src/moe_kernels.py:191-193);
     # bf16 weights under fp32 activations are widened exactly inside the kernels
     args = pack.args_for(act)
-    d_ff = experts[0].gate.out_features
+    d_ff = pack.ffn
     d_model = x.size(1)
     out = torch.empty(plan.rows, d_model, dtype=dtype, device=x.device)
     if plan.rows:

@@ -87,3 +87,39 @@ def test_pack_does_not_hold_the_experts_weights(dtype):
     layer.cpu()
     assert before - torch.cuda.memory_allocated() >= weights
     assert torch.equal(step.step(x), want)
+
+
+def layer_of(ffn, seed=0):
+    config = qa.QuantaWeaveConfig(vocab_size=2, hidden_size=64, layers=1, ffn_size=ffn, num_experts=4, top_k=2,
+                                  attention_heads=1, max_sequence_length=64)
+    torch.manual_seed(seed)
+    return qa.TopKMoE(config).cuda()
+
+
+@torch.no_grad()
+def test_calls_follow_the_weights_width():
+    """Experts whose matrices were replaced by narrower ones (pruned hidden units,
+    nn.Linear's attributes as they were) are evaluated at the width of the matrices,
+    also after a call at the old width."""
+    layer, narrow = layer_of(128), layer_of(64, seed=1)
+    x = torch.randn(1, 32, 64, device="cuda")
+    layer(x)
+    layer.router.weight.copy_(narrow.router.weight)
+    for mine, other in zip(layer.experts, narrow.experts):
+        for name in ("gate", "up", "down"):
+            getattr(mine, name).weight = torch.nn.Parameter(getattr(other, name).weight.clone())
+    assert torch.equal(layer(x)[0], narrow(x)[0])
+    counts = [10, 0, 21, 1]
+    assert torch.equal(qa.moe_kernels.grouped_swiglu(x[0], layer.experts, counts),
+                       qa.moe_kernels.grouped_swiglu(x[0], narrow.experts, counts))
+
+
+@torch.no_grad()
+def test_a_layer_pickled_by_an_earlier_release_runs():
+    """Whole-module pickles carry the module's cache of workspace sizes; entries of
+    the earlier form (four sizes per shape) are left alone."""
+    layer = layer_of(64)
+    x = torch.randn(1, 32, 64, device="cuda")
+    want = layer(x)[0]
+    layer.__dict__["_qw_sizes"] = {(32, 64, 4, 2, _lib.QW_F32): (64, 256, 256, 256)}
+    assert torch.equal(layer(x)[0], want)
