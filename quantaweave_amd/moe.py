@@ -636,26 +636,28 @@ def _router_operand(router_w: Tensor) -> Tensor:
 
 def _forward_call(flat: Tensor, act: int, router_w: Tensor, moe: TopKMoE, pack: ExpertPack, cap: int,
                   bias: Optional[Tensor]) -> dict:
-    """The whole layer forward as one qw_moe_forward call (inference)."""
+    """The whole layer forward as one qw_moe_forward_balance call (inference)."""
     dev = flat.device
     T, width = flat.shape
     E, K = moe.num_experts, moe.top_k
     R = T * K
     Rm = max(R, 1)
     rw = _router_operand(router_w)
-    # the per-call outputs in two slabs (int32 and fp32), handed out as views;
-    # the first two int32 are the 64-bit overflow count
-    ints = torch.empty(2 + R + 2 * E + 2 + 2 * Rm, dtype=torch.int32, device=dev)
-    flts = torch.empty(T * E + R + 2 + E, dtype=torch.float32, device=dev)
-    overflow, top_idx, counts, kept_counts, totals, dropped_token, dropped_expert = ints.split([2, R, E, E, 2, Rm, Rm])
-    probs, top_w, balance, zero, importance = flts.split([T * E, R, 1, 1, E])
+    # the per-call outputs in two slabs (int32 and fp32), handed out as views; the overflow
+    # count and the zero apart, for a caller who keeps them of every call
+    ints = torch.empty(R + 2 * E + 2 + 2 * Rm, dtype=torch.int32, device=dev)
+    flts = torch.empty(T * E + R + 1 + E, dtype=torch.float32, device=dev)
+    scalars = torch.empty(2, dtype=torch.int64, device=dev)
+    top_idx, counts, kept_counts, totals, dropped_token, dropped_expert = ints.split([R, E, E, 2, Rm, Rm])
+    probs, top_w, balance, importance = flts.split([T * E, R, 1, E])
     r = dict(out=torch.empty_like(flat), probs=probs.view(T, E), top_w=top_w.view(T, K), balance=balance.view(()),
              top_idx=top_idx.view(T, K), counts=counts, kept_counts=kept_counts, totals=totals,
-             dropped_token=dropped_token, dropped_expert=dropped_expert, overflow=overflow.view(torch.int64).view(()),
-             zero=zero.view(()))
+             dropped_token=dropped_token, dropped_expert=dropped_expert, overflow=scalars[0],
+             zero=scalars.view(torch.float32)[2])
     if not T:
-        ints[:2 + R + 2 * E + 2].zero_()
+        ints[:R + 2 * E + 2].zero_()
         flts.zero_()
+        scalars.zero_()
         return r
     d_ff = pack.ffn
     sizes = moe.__dict__.setdefault("_qw_sizes", {})
@@ -666,12 +668,12 @@ def _forward_call(flat: Tensor, act: int, router_w: Tensor, moe: TopKMoE, pack: 
         nbytes = sizes[key] = lib.qw_moe_forward_balance_workspace_bytes(T, width, E, K, d_ff, act)
     s = torch.cuda.current_stream(dev).cuda_stream
     wp = _stream_workspace(moe, nbytes, dev, s).data_ptr()
-    ip, fp = ints.data_ptr() + 8, flts.data_ptr()  # top_idx, probs
+    ip, fp, sp = ints.data_ptr(), flts.data_ptr(), scalars.data_ptr()
     _lib.check(lib.qw_moe_forward_balance(
         flat.data_ptr(), act, T, width, rw.data_ptr(), _hip.act_code(rw, "router"), float(moe.router_temperature),
         _hip.ptr(bias), E, K, cap, d_ff, *pack.args(), r["out"].data_ptr(), fp, ip, fp + 4 * T * E, ip + 4 * R,
         ip + 4 * (R + E), ip + 4 * (R + 2 * E), ip + 4 * (R + 2 * E + 2), ip + 4 * (R + 2 * E + 2 + Rm),
-        fp + 4 * (T * E + R + 2), fp + 4 * (T * E + R), ip - 8, fp + 4 * (T * E + R + 1), wp, nbytes, s),
+        fp + 4 * (T * E + R + 1), fp + 4 * (T * E + R), sp, sp + 8, wp, nbytes, s),
         "qw_moe_forward_balance")
     return r
 

@@ -561,6 +561,21 @@ def test_forward_balance_equals_the_stand_alone_kernels(T, E):
     assert int(got["overflow"]) == int(got["totals"][1]) and float(got["zero"]) == 0.0
 
 
+@torch.no_grad()
+@pytest.mark.parametrize("T", [0, 33, 512])
+def test_kept_scalars_hold_no_call_buffers(T):
+    """The overflow count and the domain loss of a call, kept by a caller who logs
+    them, do not keep the call's routing arrays alive."""
+    config = qa.QuantaWeaveConfig(vocab_size=2, hidden_size=64, layers=1, ffn_size=64, num_experts=8, top_k=2,
+                                  attention_heads=1, max_sequence_length=512, capacity_factor=0.5)
+    layer = qa.TopKMoE(config).cuda()
+    _, _, dropped, overflow, domain = layer(torch.randn(1, T, 64, device="cuda"))
+    for t in (dropped, overflow, domain):
+        assert t.untyped_storage().nbytes() <= 64
+    assert overflow.dtype == torch.int64 and domain.dtype == torch.float32 and not overflow.shape and not domain.shape
+    assert int(overflow) == int(layer.last_plan["totals"][1]) and float(domain) == 0.0
+
+
 def _balance_fixed_order(probs, counts, T, K, E):
     """qw_moe_balance_ws's additions in order, in float32: per 64-token chunk
     four strided sums (tokens j, j + 4, ... of the chunk) added as ((s0 + s1) + s2)
