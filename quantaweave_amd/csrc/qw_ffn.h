@@ -71,6 +71,12 @@ __device__ __forceinline__ bool xcd_tile(const XcdGrid& g, int b, int* x, int* e
   return *e < g.experts && *z < g.zs;
 }
 
+// The matrix-core kernels bring 16-byte pieces of the activations straight to LDS:
+// the rows have to start on 16 bytes (whole 64-column rows do where the bases do).
+inline bool rows_on_16_bytes(const FfnArgs& a) {
+  return ((reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.hidden)) & 15) == 0;
+}
+
 int launch_ffn_generic(const FfnArgs& a, hipStream_t stream);
 int launch_ffn_mfma(const FfnArgs& a, hipStream_t stream, bool* handled);
 int launch_ffn_quant(const FfnArgs& a, hipStream_t stream, bool* handled);

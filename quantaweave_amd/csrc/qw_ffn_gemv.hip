@@ -1365,7 +1365,8 @@ int launch_fmt(const FfnArgs& a, hipStream_t stream) {
 // Whether experts of this many rows are streamed rather than multiplied in
 // tiles.  Quantised weights: the streaming kernels multiply the exact codes, the
 // matrix-core ones rounded weights, and take over only from 16 rows.  16-bit
-// weights at widths that are no multiples of 64 have no matrix-core kernel
+// weights at widths that are no multiples of 64 (or rows off 16 bytes) have no
+// matrix-core kernel
 // (200 x 520, 12 experts of 8 rows: 18 us streamed, 73 on the general kernel; 1544
 // x 776, 16 experts of 15: 108 / 617).  Others: a streaming pass takes 4 rows of an
 // expert and reads all its weights; the matrix-core kernel reads them once
@@ -1378,7 +1379,7 @@ int launch_fmt(const FfnArgs& a, hipStream_t stream) {
 // of more than four chunks per lane (widths above 2048) stream more slowly (3072 x
 // 768, 6 experts of 5 rows 51 / 43, 4096 x 1408, one expert of 15 65 / 55).
 bool streamed(const FfnArgs& a) {
-  if (quantized(a.wfmt) || a.d_model % 64 || a.d_ff % 64) return a.avg_rows < 16;
+  if (quantized(a.wfmt) || a.d_model % 64 || a.d_ff % 64 || !rows_on_16_bytes(a)) return a.avg_rows < 16;
   if (a.avg_rows < 3 || a.avg_rows >= 16) return a.avg_rows < 3;
   const double widths = static_cast<double>(a.d_model + a.d_ff);
   const double megabytes = 6e-6 * a.d_model * a.d_ff * a.experts * (a.avg_rows + 3) / 4;  // read in all passes

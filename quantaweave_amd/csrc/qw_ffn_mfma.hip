@@ -573,7 +573,7 @@ int launch_ffn_mfma(const FfnArgs& a, hipStream_t stream, bool* handled) {
   if (!is_half(a.act)) return QW_OK;
   if (!quant && (f16 ? (a.wfmt != QW_F16 && a.wfmt != QW_F16T) : (a.wfmt != QW_BF16 && a.wfmt != QW_BF16T)))
     return QW_OK;
-  if (a.d_model % 64 || a.d_ff % 64) return QW_OK;
+  if (a.d_model % 64 || a.d_ff % 64 || !rows_on_16_bytes(a)) return QW_OK;
   if (quant && !(quant_fits(a.gate, a.wfmt) && quant_fits(a.up, a.wfmt) && quant_fits(a.down, a.wfmt))) return QW_OK;
   const int64_t rows_cap = a.row_cap > 0 ? a.row_cap : a.max_rows;
   if (quant && likely_rows(a, 2.0) <= kQuantRows) return QW_OK;  // dequantised once per weight instead of twice

@@ -664,7 +664,7 @@ int pick_sub(int64_t rows) {
 
 int launch_ffn_quant(const FfnArgs& a, hipStream_t stream, bool* handled) {
   *handled = false;
-  if (!is_half(a.act) || (a.wfmt != QW_I8 && a.wfmt != QW_U4)) return QW_OK;
+  if (!is_half(a.act) || (a.wfmt != QW_I8 && a.wfmt != QW_U4) || !rows_on_16_bytes(a)) return QW_OK;
   if (!quant_fits(a.gate, a.wfmt) || !quant_fits(a.up, a.wfmt) || !quant_fits(a.down, a.wfmt)) return QW_OK;
   const int64_t cap = a.row_cap > 0 ? a.row_cap : a.max_rows;
   const int64_t rows = likely_rows(a, 2.0);

@@ -73,3 +73,22 @@ def test_kernel_family_of_few_rows(D, F_, counts, path, dtype):
     ref = reference(x, counts, gate, up, down)
     tol = 4 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11)  # as above
     assert ((y.double() - ref).abs().max() / ref.abs().max()).item() <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,path", [(1, "stream"), (5, "stream"), (15, "stream"), (40, "generic")])
+def test_rows_that_start_off_16_bytes(rows, path, dtype):
+    """Activations at an odd element of their buffer: the kernels that copy 16-byte
+    pieces straight to LDS do not take them."""
+    torch.manual_seed(rows)
+    E, D, F_ = 9, 128, 192
+    make = lambda *s: (torch.randn(*s, device="cuda") * 0.05).to(dtype)  # noqa: E731
+    gate, up, down = make(E, F_, D), make(E, F_, D), make(E, D, F_)
+    x = torch.randn(rows * E * D + 1, device="cuda").to(dtype)[1:].view(rows * E, D)
+    assert x.data_ptr() % 16
+    offsets = torch.arange(0, rows * E + 1, rows, dtype=torch.int32, device="cuda")
+    print(f"case off 16 bytes, {rows} rows {dtype}", flush=True)
+    y = hipcall.experts(x, offsets, FMT[dtype], gate, up, down)
+    assert torch.equal(y, hipcall.experts(x.clone(), offsets, FMT[dtype], gate, up, down, path=path))
+    with pytest.raises(RuntimeError, match="do not take"):
+        hipcall.experts(x, offsets, FMT[dtype], gate, up, down, path="mfma")
