@@ -9,13 +9,17 @@
 // weight is therefore dequantised once per workgroup: a wave owns 64 weight
 // rows for all rows of the chunk (4 waves, 256 weight rows; gate/up: 32 gate
 // rows and the matching 32 up rows, so silu(g) * u is formed in registers), its
-// codes go straight from global memory to registers, two K slices ahead, and
-// only the activations are staged in LDS (a ring of three slices).  Two
-// workgroups share a compute unit, so one wave's conversions run under
-// another's MFMAs.  Against the 16-bit kernel's layout, whose eight waves
-// dequantise every weight twice: int4 layer of 64 rows per expert (T 2049, d
-// 4096, f 1408) 571 -> 350 us, int8 (d 2048, f 1024) 213 -> 156 us; the int4
-// matrix 2048 x 7168 over 1023 rows 1476 us on the general kernel -> 55 us.
+// codes go straight from global memory to registers, requested one to two K
+// slices ahead, and only the activations are staged in LDS (a ring of three
+// slices).  In the built loops of most variants the compiler adds a wait for
+// everything in flight per two slices (it moves the codes between registers on
+// the way back, or takes its own count of the loads), so the lead holds for
+// every other slice only.  Two workgroups share a compute unit, so one wave's
+// conversions run under another's MFMAs.  Against the 16-bit kernel's layout,
+// whose eight waves dequantise every weight twice: int4 layer of 64 rows per
+// expert (T 2049, d 4096, f 1408) 571 -> 346 us, int8 (d 2048, f 1024) 213 -> 151
+// us; the int4 matrix 2048 x 7168 over 1023 rows 1476 us on the general kernel
+// -> 55 us.
 // With two slices fetched together (whole 128-byte lines per request) and one
 // slice of lead: 375 us for that int4 layer, no gain.
 //
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
   const int group32 = wa.group / 32;             // MFMA steps per scale
   const int KT = K / KS;
 
-  // Codes and scales of the next two slices, in flight in registers.
+  // Codes and scales of the next two slices, requested into registers.
   uint32_t raw[2][QP_NT][DW];
   float sc[2][QP_NT];
   constexpr int BL = QP_NT * (RS ? 1 : 2);  // loads per slice
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
     auto slice = [&](int kt, auto buf) {
       constexpr int BUF = decltype(buf)::value;
       // slice kt has landed (activations in LDS, codes in registers); slice
-      // kt + 1 stays in flight.  Every slice issues the same loads (past the
+      // kt + 1 may stay in flight.  Every slice issues the same loads (past the
       // end those of the last one), so the count is fixed.
       wait_vmcnt<AL + BL>();
       ring_barrier();  // visible to every wave, and every wave is done with slice kt - 1
@@ -427,7 +431,7 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
 
 // A few rows against one quantised matrix: 16 SUB rows by 64 weight rows per
 // workgroup, its four waves taking every fourth K slice each, with codes and
-// activation operands straight in registers one slice ahead, no LDS ring and no
+// activation operands straight in registers, requested one slice ahead, no LDS ring and no
 // barrier in the K loop; the four partial tiles are added in wave order.
 // Bound by the latency of a wave's chain of slices: with 256 weight rows per
 // workgroup (the kernel above) 2048 x 7168 gives 28 workgroups of 16 or 32

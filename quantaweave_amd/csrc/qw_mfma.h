@@ -115,8 +115,9 @@ inline int64_t likely_rows(const FfnArgs& a, double sigmas) {
 // each weight once; with more, the one whose larger row chunks read fewer
 // weights.  Whole layer, this one against the other: int4 (d 4096, f 1408) 342
 // against 561 us at 64 rows per expert, 562 / 596 at 128, 646 / 660 at 188,
-// 870 / 753 at 256; int8 (d 2048, f 1024) 156 / 213, 236 / 251, 264 / 269,
-// 378 / 301 us.
+// 870 / 753 at 256; int8 (d 2048, f 1024) 151 / 213, 220 / 251, 261 / 269,
+// 378 / 301 us.  fp16 activations (expert stage): int4 308 / 463 at 64 rows, 512 /
+// 568 at 128, 553 / 596 at 160, int8 119 / 195, 193 / 225, 213 / 231.
 constexpr int64_t kQuantRows = 192;
 
 }  // namespace qw
