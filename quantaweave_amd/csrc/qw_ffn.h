@@ -20,8 +20,8 @@ struct FfnArgs {
   int64_t row_cap;           // most rows any one expert can hold (capacity bound)
   // Optional saved activations for a backward pass (act dtype, plan-ordered
   // rows): gate and up projections [max_rows, d_ff] before the SiLU, and the
-  // expert output rows [max_rows, d_model] before the row weight.  The GEMV
-  // path does not save; the MFMA and general kernels do.
+  // expert output rows [max_rows, d_model] before the row weight.  Quantised
+  // experts do not train: their streaming kernels do not save.
   void* save_gate = nullptr;
   void* save_up = nullptr;
   void* save_y = nullptr;
