@@ -149,10 +149,11 @@ __global__ __launch_bounds__(MF_THREADS) void ffn_mfma_kernel(
   // ---- tile of this workgroup (XCD-aware enumeration) ----
   const int b = blockIdx.x;
   const int xcd = b % kXcds, j = b / kXcds;
-  // XCD x takes the row chunks of experts x, x + 8, ..., each chunk's column
-  // tiles back to back.  m_chunks > 0: every expert has m_chunks chunk slots
-  // (the capacity bound is tight); m_chunks == 0: the chunks that hold rows
-  // are found on the device, so a loose bound (no capacity) costs no launches.
+  // Each chunk's column tiles back to back on one XCD.  m_chunks > 0: every
+  // expert has m_chunks chunk slots (the capacity bound is tight), those of
+  // experts x, x + 8, ... on XCD x; m_chunks < 0 (a loose bound): the chunks that
+  // hold rows are found on the device and dealt to the XCDs in runs of -m_chunks
+  // (loose_run), which share their weights in the L2.
   const int nt = j % n_tiles;
   int mc = 0, e;
   if (m_chunks > 0) {
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(MF_THREADS) void ffn_mfma_kernel(
     mc = (j / n_tiles) % m_chunks;
     if (e >= experts) return;
   } else {
-    e = find_tile(offsets, experts, max_rows, MCH, j / n_tiles, &mc, xcd, kXcds);
+    e = find_run_chunk(offsets, experts, max_rows, MCH, -m_chunks, xcd, j / n_tiles, &mc);
     if (e < 0) return;
   }
   const int e_lo = max(offsets[e], 0);
@@ -518,13 +519,13 @@ int launch_t(const void* x, const int32_t* row_index, const int32_t* offsets, in
              const MfW& wb, int n_w, int K, const float* row_weight, void* out, int n_out, int experts,
              int64_t rows_cap, void* save_a, void* save_b, hipStream_t stream) {
   const int n_tiles = static_cast<int>(ceil_div(GATEUP ? n_w : n_out, GATEUP ? MF_NB / 2 : MF_NB));
-  // chunks one XCD can own: its experts' chunks at the capacity bound, and at
-  // most all rows in chunks plus one partial chunk per expert
-  const int64_t per_xcd_experts = ceil_div(experts, kXcds);
-  const int64_t slots = per_xcd_experts * ceil_div(rows_cap, 32 * SUBT);
-  const int64_t found = ceil_div(max_rows, 32 * SUBT) + per_xcd_experts;
-  const int64_t chunks = std::min(slots, found);
-  const int m_chunks = slots <= found ? static_cast<int>(ceil_div(rows_cap, 32 * SUBT)) : 0;
+  // chunks of one XCD: its experts' slots at the capacity bound, or those its runs can hold
+  const int run = loose_run(max_rows, experts, 32 * SUBT);
+  const int64_t slots = ceil_div(experts, kXcds) * ceil_div(rows_cap, 32 * SUBT);
+  const int64_t found = loose_chunks(max_rows, experts, 32 * SUBT, run);
+  const bool fixed = slots <= ceil_div(max_rows, 32 * SUBT) + ceil_div(experts, kXcds);
+  const int64_t chunks = fixed ? slots : found;
+  const int m_chunks = fixed ? static_cast<int>(ceil_div(rows_cap, 32 * SUBT)) : -run;
   const int64_t grid = static_cast<int64_t>(kXcds) * chunks * n_tiles;
   if (grid > INT32_MAX) return set_error(QW_ERR_UNSUPPORTED, "MFMA grid too large");
   const size_t lds = static_cast<size_t>(mf_stages<WF>(SUBT)) * (32 * SUBT * MF_ROWB + MfB<WF>::STAGE);

@@ -175,9 +175,9 @@ __global__ __launch_bounds__(QP_THREADS, 2) void ffn_quant_kernel(
       nt = j / m_chunks % n_tiles;
       e = xcd + kXcds * (j / m_chunks / n_tiles);
       if (e >= experts) return;
-    } else {  // a loose bound: the chunks that hold rows are found here
+    } else {  // a loose bound: the chunks that hold rows are found here, in runs of -m_chunks on one XCD
       nt = j % n_tiles;
-      e = find_tile(offsets, experts, max_rows, MCH, j / n_tiles, &mc, xcd, kXcds);
+      e = find_run_chunk(offsets, experts, max_rows, MCH, -m_chunks, xcd, j / n_tiles, &mc);
       if (e < 0) return;
     }
   } else {
@@ -597,18 +597,18 @@ int launch_t(const QpArgs& a, hipStream_t stream) {
   int64_t grid;
   int m_chunks;
   if (a.experts >= kXcds) {
-    // chunks one XCD can own: its experts' chunks at the row bound, and at
-    // most all rows in chunks plus one partial chunk per expert
-    const int64_t per_xcd = ceil_div(a.experts, kXcds);
-    const int64_t slots = per_xcd * ceil_div(a.row_cap, MCH);
-    const int64_t found = ceil_div(a.max_rows, MCH) + per_xcd;
+    // chunks of one XCD: its experts' slots at the row bound, or those its runs can hold
+    const int run = loose_run(a.max_rows, a.experts, MCH);
+    const int64_t slots = ceil_div(a.experts, kXcds) * ceil_div(a.row_cap, MCH);
+    const int64_t found = loose_chunks(a.max_rows, a.experts, MCH, run);
     // Where the bound allows a chunk that few experts fill, the chunks are found
     // on the device too: as fixed slots, the rare ones started between empty
     // ones and ran into a last round of their own (int4 layer, T = 2500, 79
     // rows per expert, capacity 98, chunks of 96 rows: 566 us against 397).
     const bool tight = ceil_div(a.row_cap, MCH) == ceil_div(a.rows, MCH);
-    m_chunks = tight && slots <= found ? static_cast<int>(ceil_div(a.row_cap, MCH)) : 0;
-    grid = static_cast<int64_t>(kXcds) * (m_chunks > 0 ? slots : std::min(slots, found)) * n_tiles;
+    const bool fixed = tight && slots <= ceil_div(a.max_rows, MCH) + ceil_div(a.experts, kXcds);
+    m_chunks = fixed ? static_cast<int>(ceil_div(a.row_cap, MCH)) : -run;
+    grid = static_cast<int64_t>(kXcds) * (fixed ? slots : found) * n_tiles;
   } else {
     m_chunks = static_cast<int>(ceil_div(a.row_cap, MCH));
     grid = static_cast<int64_t>(kXcds) * ceil_div(static_cast<int64_t>(a.experts) * n_tiles, kXcds) * m_chunks;

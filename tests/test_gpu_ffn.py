@@ -531,3 +531,41 @@ def test_prefill_hidden_rows_follow_the_reference_rounding():
     equal = float(np.mean(ulps == 0))
     print(f"  {ulps.size} hidden values: {equal:.6f} equal, max {int(ulps.max())} ulp", flush=True)
     assert int(ulps.max()) <= 1 and equal >= 0.999
+
+
+@pytest.mark.parametrize("fmt", ["bf16", "int8", "int4"])
+@pytest.mark.parametrize("counts", [
+    [0, 0, 1000] + [0] * 6, [700, 0, 5, 300, 1, 0, 64, 65, 63], [33] * 70 + [900], [20] * 200,
+    [400] * 3 + [0] * 5 + [7] * 130,
+])
+def test_loose_row_bound_visits_every_row(fmt, counts):
+    """Without a bound on an expert's rows its chunks are found on the device and
+    dealt over the XCDs in runs: the same bits as each expert on its own, for one
+    popular expert, many small ones and more than a wave of them."""
+    torch.manual_seed(len(counts))
+    E, D, F_, rows = len(counts), 128, 192, sum(counts)
+    offsets = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32, device="cuda")
+    x = torch.randn(rows, D, device="cuda").bfloat16()
+
+    def matrices(out, cols):
+        if fmt == "bf16":
+            return (torch.randn(E, out, cols, device="cuda") * 0.05).bfloat16(), None
+        if fmt == "int8":
+            return (torch.randint(-127, 128, (E, out, cols), device="cuda", dtype=torch.int8),
+                    torch.rand(E, out, 1, device="cuda") * 1e-3)
+        return (torch.randint(0, 256, (E, out, cols // 2), device="cuda", dtype=torch.uint8),
+                torch.rand(E, out, cols // 32, device="cuda") * 1e-2)
+
+    (gate, gs), (up, us), (down, ds) = matrices(F_, D), matrices(F_, D), matrices(D, F_)
+    code = {"bf16": _lib.QW_BF16, "int8": _lib.QW_I8, "int4": _lib.QW_U4}[fmt]
+    groups = {"bf16": (0, 0), "int8": (D, F_), "int4": (32, 32)}[fmt]
+    print(f"case {fmt} {E} experts {rows} rows", flush=True)
+    loose = H.experts(x, offsets, code, gate, up, down, gs, us, ds, *groups, path="mfma")
+    own = lambda t, e: None if t is None else t[e:e + 1]  # noqa: E731
+    first = 0
+    for e, n in enumerate(counts):
+        if n:
+            alone = H.experts(x[first:first + n], torch.tensor([0, n], dtype=torch.int32, device="cuda"), code,
+                              *(own(t, e) for t in (gate, up, down, gs, us, ds)), *groups, path="mfma")
+            assert torch.equal(loose[first:first + n], alone), e
+        first += n
