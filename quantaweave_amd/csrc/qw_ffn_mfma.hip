@@ -54,9 +54,10 @@
 // weights is made.
 //
 // Workgroup -> tile order is XCD-aware: workgroups are dispatched round-robin
-// over the 8 XCDs, so block b runs on XCD b%8; all tiles of one expert are
-// given to one XCD and enumerated column-fastest, which keeps the expert's
-// activation rows (and a second row chunk's weights) in that XCD's L2.
+// over the 8 XCDs, so block b runs on XCD b%8; all tiles of one expert (of a run
+// of its chunks, where the row bound is loose) are given to one XCD and
+// enumerated column-fastest, which keeps the expert's activation rows (and a
+// second row chunk's weights) in that XCD's L2.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
